@@ -674,23 +674,153 @@ int launch_attn_split(const AttnArgs& a, int nsplit, int heads, hipStream_t s, i
   return fw_check_launch("attention split");
 }
 
-// Merges the split results of one head; splits with l == 0 are empty and skipped.
+// Merges the split results of one head; splits with l == 0 are empty and skipped. A lane's values of
+// kCombineBatch splits are requested together: one at a time behind a branch each, the 7 splits of a
+// 448-key cache were 7 round trips to L2 in a row (4.6 us a launch for 20 waves of work).
+constexpr int kCombineBatch = 8;
+
 __global__ void __launch_bounds__(64) attn_combine_kernel(AttnArgs a, int nsplit) {
   const int head = blockIdx.x, d = threadIdx.x;
   const float* pm = a.part_m + head * nsplit;
   const float* pl = a.part_l + head * nsplit;
   const float* pa = a.part_acc + static_cast<size_t>(head) * nsplit * kHeadDim;
   float m = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) m = fmaxf(m, pm[s]);
+  for (int s0 = 0; s0 < nsplit; s0 += kCombineBatch) {
+    float v[kCombineBatch];
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) v[i] = pm[min(s0 + i, nsplit - 1)];
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) m = fmaxf(m, v[i]);
+  }
   float num = 0.f, den = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    if (pl[s] > 0.f) {
-      const float wgt = __expf(pm[s] - m);
-      num = fmaf(pa[s * kHeadDim + d], wgt, num);
-      den = fmaf(pl[s], wgt, den);
+  for (int s0 = 0; s0 < nsplit; s0 += kCombineBatch) {
+    float vm[kCombineBatch], vl[kCombineBatch], va[kCombineBatch];
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) {
+      const int sp = min(s0 + i, nsplit - 1);
+      vm[i] = pm[sp];
+      vl[i] = pl[sp];
+      va[i] = pa[sp * kHeadDim + d];
+    }
+#pragma unroll
+    for (int i = 0; i < kCombineBatch; ++i) {
+      const float wgt = __expf(vm[i] - m);
+      const bool live = s0 + i < nsplit && vl[i] > 0.f;  // an empty split's acc may hold anything
+      num = live ? fmaf(va[i], wgt, num) : num;
+      den = live ? fmaf(vl[i], wgt, den) : den;
     }
   }
   a.out[head * kHeadDim + d] = f2h(num / den);
+}
+
+// ------------------------------------------------------------------------------------------
+// decode_attention for caches of up to kDirectKeys keys in one launch: one block per head computes the
+// 64-key splits' wave partials (attn_split_kernel<2>'s: 4 waves of 16 keys a split), merges each split
+// (split_merge) and combines the splits (attn_combine_kernel), all through LDS, so the output is that of
+// the two launches bit for bit. Latency bounds it: 20 blocks of at most 112 KB each. What it saves is the
+// second launch and the partials' trip through memory (448-key cache, 224 keys filled, 20 heads: 4.2 us in
+// the kernel trace against 2.9 + 4.6 us for the two launches). Keys below kDirectFirst are requested before the length is known; the rest, which a
+// cache filled no further does not need, once it is. Longer caches keep the split grid: one CU would
+// read a 1500-key head (384 KB) in about 5 us, which takes 24 blocks 1 us.
+// ------------------------------------------------------------------------------------------
+constexpr int kDirectWaves = 16, kDirectKeys = 512;
+constexpr int kDirectFirst = kDirectWaves * 16;  // keys of the first round: 16 per wave
+constexpr int kDirectRounds = kDirectKeys / kDirectFirst;
+constexpr int kDirectSplits = kDirectKeys / kSplitKeys;
+static_assert(kDirectFirst % kSplitKeys == 0 && kDirectKeys % kDirectFirst == 0, "whole splits per round");
+
+__global__ void __launch_bounds__(kDirectWaves * 64) attn_direct_kernel(AttnArgs a) {
+  __shared__ float wm[kDirectSplits * 4], wl[kDirectSplits * 4];
+  __shared__ float wacc[kDirectSplits * 4][kHeadDim];
+  __shared__ float sm[kDirectSplits], sl[kDirectSplits], sacc[kDirectSplits][kHeadDim];
+  const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ks = lane >> 3, c = lane & 7;
+  const size_t hoff = static_cast<size_t>(head) * a.max_len * kHeadDim;
+  _Float16* kh = a.k + hoff;
+  _Float16* vh = a.v + hoff;
+  const int64_t pos_raw = a.len_state ? a.len_state[0] : 0;
+  const uint4 qc = reinterpret_cast<const uint4*>(a.q + head * kHeadDim)[c];
+  uint4 knew = make_uint4(0, 0, 0, 0), vnew = make_uint4(0, 0, 0, 0);
+  if (a.k_new) {
+    knew = reinterpret_cast<const uint4*>(a.k_new + head * kHeadDim)[c];
+    vnew = reinterpret_cast<const uint4*>(a.v_new + head * kHeadDim)[c];
+  }
+  uint4 kr[2], vr[2];
+  auto request = [&](int w0) {  // the wave's 16 keys from w0 on; keys past the cache load its last row
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const size_t j = static_cast<size_t>(min(w0 + p * 8 + ks, a.max_len - 1));
+      kr[p] = reinterpret_cast<const uint4*>(kh + j * kHeadDim)[c];
+      vr[p] = reinterpret_cast<const uint4*>(vh + j * kHeadDim)[c];
+    }
+  };
+  request(wave * 16);
+  const int pos = a.len_state ? static_cast<int>(pos_raw < 0 ? 0 : (pos_raw >= a.max_len ? a.max_len - 1 : pos_raw)) : -1;
+  const int len = a.len_state ? pos + 1 : a.max_len;
+  const int nsplit = (len + kSplitKeys - 1) / kSplitKeys;  // splits that hold keys
+#pragma unroll
+  for (int r = 0; r < kDirectRounds; ++r) {
+    const int w0 = r * kDirectFirst + wave * 16, slot = r * kDirectWaves + wave;
+    if (slot / 4 < nsplit) {  // wave-uniform; waves of one split agree
+      if (r > 0) request(w0);
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        if (a.k_new && w0 + p * 8 + ks == pos) {  // the new row replaces the (stale) cached one
+          kr[p] = knew;
+          vr[p] = vnew;
+        }
+      split_wave_partial<2>(kr, vr, qc, w0, min(w0 + 16, len), a.scale, wm + slot, wl + slot, wacc[slot]);
+    }
+  }
+  if (a.k_new && tid < 16) {  // a lane that holds chunk c of the new row stores it
+    if (tid < 8)
+      reinterpret_cast<uint4*>(kh + static_cast<size_t>(pos) * kHeadDim)[c] = knew;
+    else
+      reinterpret_cast<uint4*>(vh + static_cast<size_t>(pos) * kHeadDim)[c] = vnew;
+  }
+  __syncthreads();
+  if (wave < nsplit) {  // one wave per split (kDirectSplits <= kDirectWaves)
+    float m, l, o;
+    split_merge<4>(wm + 4 * wave, wl + 4 * wave, wacc + 4 * wave, lane, m, l, o);
+    sacc[wave][lane] = o;
+    if (lane == 0) {
+      sm[wave] = m;
+      sl[wave] = l;
+    }
+  }
+  __syncthreads();
+  if (tid >= kHeadDim) return;
+  float vm[kDirectSplits], vl[kDirectSplits], va[kDirectSplits], m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kDirectSplits; ++i) {
+    const int sp = min(i, nsplit - 1);
+    vm[i] = sm[sp];
+    vl[i] = sl[sp];
+    va[i] = sacc[sp][tid];
+  }
+#pragma unroll
+  for (int i = 0; i < kDirectSplits; ++i) m = fmaxf(m, vm[i]);
+  float num = 0.f, den = 0.f;
+#pragma unroll
+  for (int i = 0; i < kDirectSplits; ++i) {
+    const float wgt = __expf(vm[i] - m);
+    const bool live = i < nsplit && vl[i] > 0.f;
+    num = live ? fmaf(va[i], wgt, num) : num;
+    den = live ? fmaf(vl[i], wgt, den) : den;
+  }
+  a.out[head * kHeadDim + tid] = f2h(num / den);
+}
+
+// The 64-key splits and their combine: one launch while a head's keys fit one block's two rounds.
+int launch_decode_attention(const AttnArgs& a, int nsplit, int heads, hipStream_t s) {
+  if (a.max_len <= kDirectKeys) {
+    hipLaunchKernelGGL(attn_direct_kernel, dim3(heads), dim3(kDirectWaves * 64), 0, s, a);
+    return fw_check_launch("decode_attention");
+  }
+  const int rc = launch_attn_split(a, nsplit, heads, s);
+  if (rc != FW_OK) return rc;
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(heads), dim3(kHeadDim), 0, s, a, nsplit);
+  return fw_check_launch("decode_attention combine");
 }
 
 // ------------------------------------------------------------------------------------------
@@ -930,10 +1060,7 @@ extern "C" int fw_decode_attention(const void* q, void* k, void* v, void* out, c
   a.part_m = part_m;
   a.part_l = part_l;
   a.part_acc = part_acc;
-  rc = launch_attn_split(a, nsplit, heads, stream);
-  if (rc != FW_OK) return rc;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(heads), dim3(kHeadDim), 0, stream, a, nsplit);
-  return fw_check_launch("decode_attention combine");
+  return launch_decode_attention(a, nsplit, heads, stream);
 }
 
 extern "C" int fw_decode_attention_fused(const void* q, void* k, void* v, void* out, const int64_t* len_state,
@@ -1214,8 +1341,5 @@ extern "C" int fw_decode_attention_noalloc(const void* q, void* k, void* v, void
   a.part_m = ws;
   a.part_l = ws + FW_NOALLOC_ATTN_SLOTS;
   a.part_acc = ws + 2 * FW_NOALLOC_ATTN_SLOTS;
-  rc = launch_attn_split(a, nsplit, heads, stream);
-  if (rc != FW_OK) return rc;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(heads), dim3(kHeadDim), 0, stream, a, nsplit);
-  return fw_check_launch("decode_attention_noalloc combine");
+  return launch_decode_attention(a, nsplit, heads, stream);
 }

@@ -167,6 +167,33 @@ def test_cross_attention(ext, hip_device, max_len, fused):
     close_rel(np32(out), ref)
 
 
+@pytest.mark.parametrize('max_len,length', [(1, 1), (17, 16), (65, 65), (256, 256), (257, 257), (512, 255), (512, 256),
+                                            (512, 257), (512, 512), (513, 513)])
+@pytest.mark.parametrize('own', [True, False])
+def test_decode_attention_one_launch_edges(ext, hip_device, max_len, length, own):
+    """Caches around the one-launch form's edges (a wave's 16 keys, a 64-key split, the 256 keys of a round,
+    the 512-key limit and past it) against the oracle; keys past the length are NaN in the cache, so a key
+    that is read as live shows."""
+    from flash_whisper_amd.selftest import workspace
+
+    rng = np.random.default_rng(max_len + length)
+    dev, heads, pos = hip_device, 3, length - 1
+    q, k, v = _attn_inputs(rng, heads, max_len)
+    q = np.float16(q.astype(np.float32) * 2)
+    k_new, v_new = np.float16(rng.standard_normal((heads, 64))), np.float16(rng.standard_normal((heads, 64)))
+    n = length if own else max_len
+    k[:, n:] = v[:, n:] = np.nan
+    tk, tv = h16(k, dev), h16(v, dev)
+    out = torch.empty(heads * 64, dtype=torch.float16, device=dev)
+    new = (torch.tensor([pos, 0], device=dev), h16(k_new, dev), h16(v_new, dev)) if own else (None, None, None)
+    ext.decode_attention(h16(q, dev), tk, tv, out, *new, *workspace(heads, -(-max_len // 64)), 0.125)
+    if own:
+        k[:, pos], v[:, pos] = k_new, v_new
+    ref = odec.attention(q.reshape(heads, 64).astype(np.float32), k[:, :n], v[:, :n], n, 0.125)
+    close_rel(np32(out), ref)
+    assert np.array_equal(tk.cpu().numpy(), k, equal_nan=True) and np.array_equal(tv.cpu().numpy(), v, equal_nan=True)
+
+
 def _lm_setup(dev, seed=4):
     from flash_whisper_amd import weights
 

@@ -6,12 +6,13 @@
 //   final:  max(x, global_max - 8), (x + 4) / 4
 // Prepare (one block, once per filterbank): the twiddle table exp(-2 pi i n / 400) built in fp64, and
 // the compacted filterbank (each mel's triangle is a short run of bins: its first bin, the run length
-// and the run's weights). Frames (one block per 12 frames): stages the reflect-padded samples in LDS,
-// applies the window, and takes each frame's 400-point real DFT as a 200-point complex FFT of the
-// (even, odd) sample pairs (Stockham autosort, radices 8, 5, 5, natural order out) followed by the
-// real-input split; then the power, the compacted filterbank (the same terms in the same order as the
-// dense product, whose other terms are zero), log10 and one block maximum. Finalize reduces the block
-// maxima, clamps, rescales and writes the fp16 time-major copy the encoder's conv stem reads.
+// and the run's weights, weight j of every mel side by side). Frames (one wave per frame): reads the
+// frame's samples (reflect-padded at the clip's ends), applies the window, and takes the 400-point real
+// DFT as a 200-point complex FFT of the (even, odd) sample pairs (Stockham autosort, radices 8, 5, 5,
+// natural order out) followed by the real-input split; then the power, the compacted filterbank (the
+// same terms in the same order as the dense product, whose other terms are zero), log10 and one block
+// maximum. Finalize reduces the block maxima, clamps, rescales and writes the fp16 time-major copy the
+// encoder's conv stem reads.
 #include <algorithm>
 #include <cstring>
 #include "fw_common.h"
@@ -21,11 +22,10 @@ namespace {
 
 constexpr int kNfft = 400, kHop = 160, kBins = 201, kMels = 128;
 constexpr int kHalf = kNfft / 2;  // complex FFT length
-constexpr int kFramesPerBlock = 12;
-constexpr int kSpan = (kFramesPerBlock - 1) * kHop + kNfft;  // samples staged per block
+constexpr int kFramesPerBlock = 12;  // one wave each
 constexpr int kRun = 16;  // longest compacted filter run; longer ones are read from the dense filters
 // Workspace layout (floats): the twiddles (float2 x 400), per mel {first bin, run length} (int2 x 128),
-// per mel kRun weights, then one maximum per frames block. The prepared part does not depend on the
+// kRun weights x 128 mels, then one maximum per frames block. The prepared part does not depend on the
 // number of samples.
 constexpr int kWsTw = 0, kWsRange = kWsTw + 2 * kNfft, kWsW = kWsRange + 2 * kMels, kWsMax = kWsW + kMels * kRun;
 static_assert(kWsRange % 2 == 0 && kWsMax % 4 == 0, "float2 / int2 / 16-byte alignment of the workspace parts");
@@ -64,11 +64,10 @@ __global__ void __launch_bounds__(1024) logmel_prepare_kernel(const float* __res
   const int first = hi < 0 ? 0 : lo;
   if (part == 0) reinterpret_cast<int2*>(ws + kWsRange)[m] = make_int2(first, len);
   float* w = ws + kWsW;
-  for (int j = part; j < kRun; j += 8) w[m * kRun + j] = (j < len && len <= kRun) ? filters[(first + j) * kMels + m] : 0.f;
+  for (int j = part; j < kRun; j += 8) w[j * kMels + m] = (j < len && len <= kRun) ? filters[(first + j) * kMels + m] : 0.f;
 }
 
-// torch.stft reflect padding (valid for |overhang| < n). Samples staged for frames past the last one
-// can overhang further; they are never used, so the index is only clamped into the buffer.
+// torch.stft reflect padding (valid for |overhang| < n); the index is clamped into the buffer besides.
 __device__ __forceinline__ int reflect(int i, int n) {
   if (i < 0) i = -i;
   if (i >= n) i = 2 * (n - 1) - i;
@@ -126,106 +125,173 @@ __device__ __forceinline__ void dft(float2 (&v)[R]) {
   else dft5(v);
 }
 
-// One Stockham stage of the 200-point FFT for every frame of the block: butterfly j of a frame reads
-// src[j + r * 200 / R], applies the twiddles exp(-2 pi i (j mod NS) r / (NS R)) (table index
-// (j mod NS) r 400 / (NS R) < 400), runs the radix-R DFT and writes dst[(j / NS) NS R + j mod NS + r NS].
+// Element i of a frame's FFT buffer in LDS: one float2 of padding every 8, so that the radix-8 stage's
+// writes (8 elements apart from lane to lane) spread over the banks.
+__device__ __forceinline__ int fft_at(int i) { return i + (i >> 3); }
+constexpr int kFftBuf = kHalf + kHalf / 8;
+
+// LDS hand-off between the lanes of one wave: its LDS accesses complete in order, so only the compiler
+// has to keep them in order.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A radix-R Stockham butterfly j of the 200-point FFT: v[r] is element j + r * 200 / R; applies the
+// twiddles exp(-2 pi i (j mod NS) r / (NS R)) (table index (j mod NS) r 400 / (NS R) < 400), runs the
+// radix-R DFT and writes dst[(j / NS) NS R + j mod NS + r NS].
 template <int R, int NS>
-__device__ __forceinline__ void fft_stage(const float2 (*src)[kHalf], float2 (*dst)[kHalf], const float2* tw, int tid) {
-  constexpr int kB = kHalf / R, kStep = kNfft / (NS * R);
+__device__ __forceinline__ void fft_butterfly(float2 (&v)[R], float2* dst, const float2* tw, int j) {
+  constexpr int kStep = kNfft / (NS * R);
   static_assert(kHalf % R == 0 && kNfft % (NS * R) == 0 && (NS - 1) * (R - 1) * kStep < kNfft, "stage shape");
-  for (int i = tid; i < kFramesPerBlock * kB; i += 256) {
-    const int f = i / kB, j = i - f * kB;
+  if constexpr (NS > 1) {
+    const int a = (j % NS) * kStep;
+#pragma unroll
+    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[a * r]);
+  }
+  dft<R>(v);
+  const int base = (j / NS) * NS * R + j % NS;
+#pragma unroll
+  for (int r = 0; r < R; ++r) dst[fft_at(base + r * NS)] = v[r];
+}
+template <int R, int NS>
+__device__ __forceinline__ void fft_stage(const float2* src, float2* dst, const float2* tw, int lane) {
+  constexpr int kB = kHalf / R;
+  static_assert(kB <= kWave, "one butterfly per lane");
+  if (lane < kB) {
     float2 v[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[r] = src[f][j + r * kB];
-    if constexpr (NS > 1) {
-      const int a = (j % NS) * kStep;
-#pragma unroll
-      for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[a * r]);
-    }
-    dft<R>(v);
-    const int base = (j / NS) * NS * R + j % NS;
-#pragma unroll
-    for (int r = 0; r < R; ++r) dst[f][base + r * NS] = v[r];
+    for (int r = 0; r < R; ++r) v[r] = src[fft_at(lane + r * kB)];
+    fft_butterfly<R, NS>(v, dst, tw, lane);
   }
 }
 
-__global__ void __launch_bounds__(256) logmel_frames_kernel(const float* __restrict__ wave, int n_samples,
-                                                            int n_frames, const float* __restrict__ filters,
-                                                            const float* __restrict__ ws, float* __restrict__ out,
-                                                            float* __restrict__ block_max) {
-  __shared__ float xs[kSpan];
-  __shared__ float2 tw[kNfft];
-  __shared__ float2 za[kFramesPerBlock][kHalf];
-  __shared__ float2 zb[kFramesPerBlock][kHalf];
-  __shared__ __align__(16) float pw[kBins][kFramesPerBlock];
-  __shared__ int2 mrange[kMels];
-  __shared__ float mw[kMels * kRun];
-  __shared__ float red[4];
-  const int tid = threadIdx.x;
-  const int f0 = blockIdx.x * kFramesPerBlock;
-  const int s0 = f0 * kHop - kNfft / 2;
+typedef float sample_pair __attribute__((ext_vector_type(2), aligned(4)));  // a waveform need not be 8-byte aligned
 
-  for (int i = tid; i < kSpan; i += 256) xs[i] = wave[reflect(s0 + i, n_samples)];
-  for (int i = tid; i < kNfft; i += 256) tw[i] = reinterpret_cast<const float2*>(ws + kWsTw)[i];
-  if (tid < kMels) mrange[tid] = reinterpret_cast<const int2*>(ws + kWsRange)[tid];
-  for (int i = tid; i < kMels * kRun; i += 256) mw[i] = ws[kWsW + i];
-  __syncthreads();
-  // z[m] = (x[2m], x[2m + 1]) windowed; periodic Hann 0.5 - 0.5 cos(2 pi n / 400)
-  for (int i = tid; i < kFramesPerBlock * kHalf; i += 256) {
-    const int f = i / kHalf, m = i - f * kHalf, n = 2 * m;
-    const float w0 = 0.5f - 0.5f * tw[n].x, w1 = 0.5f - 0.5f * tw[n + 1].x;
-    za[f][m] = make_float2(xs[f * kHop + n] * w0, xs[f * kHop + n + 1] * w1);
+// One wave per frame and no block barrier between the FFT stages: latency bounds the kernel (a frame is
+// 7 kFLOP over five LDS exchanges), so it wants several independent waves on each SIMD. For 30 s, 250
+// blocks of 12 waves, which share one copy of the tables: 7.2 us in the kernel trace (16 waves 7.8, 8
+// waves 8.0, 6 waves 7.9, 4 waves 8.4, 2 waves 9.5). The form before it took the same 12 frames with 4
+// waves, one a SIMD, a barrier after each stage and LDS strides that met in 16 of the 64 banks: 12.4 us.
+__global__ void __launch_bounds__(kFramesPerBlock * 64) logmel_frames_kernel(const float* __restrict__ wave_in,
+                                                                             int n_samples, int n_frames,
+                                                                             const float* __restrict__ filters,
+                                                                             const float* __restrict__ ws,
+                                                                             float* __restrict__ out,
+                                                                             float* __restrict__ block_max) {
+  constexpr int kThreads = kFramesPerBlock * 64;
+  __shared__ float2 tw[kNfft];
+  __shared__ float2 bufs[kFramesPerBlock][2][kFftBuf];
+  __shared__ float pws[kFramesPerBlock][kBins];
+  __shared__ float mw[kRun * kMels];
+  __shared__ float tile[kMels][kFramesPerBlock + 1];
+  __shared__ float red[kFramesPerBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int f0 = blockIdx.x * kFramesPerBlock;
+  const int f = min(f0 + wave, n_frames - 1);  // a wave past the end repeats the last frame and stores nothing
+  const int s0 = f * kHop - kNfft / 2;
+  float2* za = bufs[wave][0];
+  float2* zb = bufs[wave][1];
+  float* pw = pws[wave];
+
+  // this lane's radix-8 inputs z[m] = (x[2m], x[2m + 1]), m = lane + 25 r
+  constexpr int kB8 = kHalf / 8;
+  float2 z[8];
+  if (s0 >= 0 && s0 + kNfft <= n_samples) {  // wave-uniform
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const sample_pair v = *reinterpret_cast<const sample_pair*>(wave_in + s0 + 2 * (min(lane, kB8 - 1) + kB8 * r));
+      z[r] = make_float2(v.x, v.y);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int i = s0 + 2 * (min(lane, kB8 - 1) + kB8 * r);
+      z[r] = make_float2(wave_in[reflect(i, n_samples)], wave_in[reflect(i + 1, n_samples)]);
+    }
   }
+  for (int i = tid; i < kNfft; i += kThreads) tw[i] = reinterpret_cast<const float2*>(ws + kWsTw)[i];
+  for (int i = tid; i < kMels * kRun / 4; i += kThreads)
+    reinterpret_cast<float4*>(mw)[i] = reinterpret_cast<const float4*>(ws + kWsW)[i];
+  const int2 rg[2] = {reinterpret_cast<const int2*>(ws + kWsRange)[lane],
+                      reinterpret_cast<const int2*>(ws + kWsRange)[lane + 64]};
   __syncthreads();
-  fft_stage<8, 1>(za, zb, tw, tid);
-  __syncthreads();
-  fft_stage<5, 8>(zb, za, tw, tid);
-  __syncthreads();
-  fft_stage<5, 40>(za, zb, tw, tid);
-  __syncthreads();
+  if (lane < kB8) {  // periodic Hann 0.5 - 0.5 cos(2 pi n / 400), then the first stage
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int n = 2 * (lane + kB8 * r);
+      const float w0 = 0.5f - 0.5f * tw[n].x, w1 = 0.5f - 0.5f * tw[n + 1].x;
+      z[r] = make_float2(z[r].x * w0, z[r].y * w1);
+    }
+    fft_butterfly<8, 1>(z, zb, tw, lane);
+  }
+  wave_lds_sync();
+  fft_stage<5, 8>(zb, za, tw, lane);
+  wave_lds_sync();
+  fft_stage<5, 40>(za, zb, tw, lane);
+  wave_lds_sync();
   // X[k] = E[k] + exp(-2 pi i k / 400) O[k] with E = (Z[k] + conj Z[200 - k]) / 2 and
   // O = (Z[k] - conj Z[200 - k]) / 2i, indices mod 200; power |X[k]|^2.
-  for (int i = tid; i < kFramesPerBlock * kBins; i += 256) {
-    const int f = i / kBins, k = i - f * kBins;
-    const float2 zk = zb[f][k % kHalf], zc = zb[f][(kHalf - k) % kHalf];
-    const float2 e = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y - zc.y));
-    const float2 o = make_float2(0.5f * (zk.y + zc.y), -0.5f * (zk.x - zc.x));
-    const float2 x = cadd(e, cmul(tw[k], o));
-    pw[k][f] = x.x * x.x + x.y * x.y;
-  }
-  __syncthreads();
-
-  // filterbank: the nonzero terms of filters^T @ power in increasing bin order, as the dense sum
-  constexpr int kF = kFramesPerBlock / 2;  // 2 groups of frames per mel
-  const int m = tid & (kMels - 1), fh = tid >> 7;
-  float acc[kF];
 #pragma unroll
-  for (int f = 0; f < kF; ++f) acc[f] = 0.f;
-  const int2 rg = mrange[m];
-  for (int j = 0; j < rg.y; ++j) {
-    const int k = rg.x + j;
-    const float fk = rg.y <= kRun ? mw[m * kRun + j] : filters[k * kMels + m];
-    if (fk != 0.f) {
-#pragma unroll
-      for (int f = 0; f < kF; ++f) acc[f] = fmaf(fk, pw[k][fh * kF + f], acc[f]);
+  for (int p = 0; p < (kBins + 63) / 64; ++p) {
+    const int k = lane + 64 * p;
+    if (k < kBins) {
+      const float2 zk = zb[fft_at(k == kHalf ? 0 : k)], zc = zb[fft_at(k == 0 || k == kHalf ? 0 : kHalf - k)];
+      const float2 e = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y - zc.y));
+      const float2 o = make_float2(0.5f * (zk.y + zc.y), -0.5f * (zk.x - zc.x));
+      const float2 x = cadd(e, cmul(tw[k], o));
+      pw[k] = x.x * x.x + x.y * x.y;
     }
   }
+  wave_lds_sync();
+
+  // filterbank: the nonzero terms of filters^T @ power in increasing bin order, as the dense sum; a lane
+  // takes mels lane and lane + 64
   float vmax = -INFINITY;
 #pragma unroll
-  for (int f = 0; f < kF; ++f) {
-    const int t = f0 + fh * kF + f;
-    if (t < n_frames) {
-      const float v = log10f(fmaxf(acc[f], 1e-10f));
-      out[static_cast<size_t>(m) * n_frames + t] = v;
-      vmax = fmaxf(vmax, v);
+  for (int h = 0; h < 2; ++h) {
+    const int m = lane + 64 * h;
+    float acc = 0.f;
+    if (rg[h].y <= kRun) {
+      for (int j = 0; j < rg[h].y; j += 4) {
+        float fk[4], pk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {  // weights past the run are zero
+          fk[e] = mw[(j + e) * kMels + m];
+          pk[e] = pw[min(rg[h].x + j + e, kBins - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = fk[e] != 0.f ? fmaf(fk[e], pk[e], acc) : acc;
+      }
+    } else {
+      for (int j = 0; j < rg[h].y; ++j) {
+        const int k = rg[h].x + j;
+        const float fk = filters[k * kMels + m];
+        if (fk != 0.f) acc = fmaf(fk, pw[k], acc);
+      }
     }
+    const float v = log10f(fmaxf(acc, 1e-10f));
+    tile[m][wave] = v;
+    vmax = fmaxf(vmax, v);
   }
   vmax = group_max<kWave>(vmax);
-  if ((tid & 63) == 0) red[tid >> 6] = vmax;
+  if (lane == 0) red[wave] = vmax;
   __syncthreads();
-  if (tid == 0) block_max[blockIdx.x] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  // each mel's frames of the block as one run
+#pragma unroll
+  for (int i = tid; i < kMels * kFramesPerBlock; i += kThreads) {
+    const int m = i / kFramesPerBlock, t = i % kFramesPerBlock;
+    if (f0 + t < n_frames) out[static_cast<size_t>(m) * n_frames + f0 + t] = tile[m][t];
+  }
+  if (tid == 0) {
+    float b = red[0];
+#pragma unroll
+    for (int w = 1; w < kFramesPerBlock; ++w) b = fmaxf(b, red[w]);
+    block_max[blockIdx.x] = b;
+  }
 }
+static_assert(kRun % 4 == 0, "the filterbank loop takes four weights at a time");
 
 constexpr int kTileT = 16;                     // frames per finalize block
 constexpr int kFinPer = kMels * kTileT / 256;  // values per thread
@@ -296,7 +362,7 @@ extern "C" int fw_log_mel_run(const float* wave, int n_samples, const float* fil
   if (ws_floats < need) return fw_fail(FW_EINVAL, "log_mel: workspace needs %lld floats", static_cast<long long>(need));
   if (reinterpret_cast<uintptr_t>(ws) & 15u) return fw_fail(FW_EINVAL, "log_mel: ws must be 16-byte aligned");
   float* maxima = ws + fw::kWsMax;
-  hipLaunchKernelGGL(fw::logmel_frames_kernel, dim3(blocks), dim3(256), 0, stream, wave, n_samples, n_frames, filters,
+  hipLaunchKernelGGL(fw::logmel_frames_kernel, dim3(blocks), dim3(fw::kFramesPerBlock * 64), 0, stream, wave, n_samples, n_frames, filters,
                      ws, out, maxima);
   int rc = fw_check_launch("log_mel frames");
   if (rc != FW_OK) return rc;

@@ -340,3 +340,22 @@ def test_encoder_product_sequence_vs_oracle(ext, hip_device):
     v = oenc.linear_op(enc, params[f'{pre}.v_proj.weight'], params[f'{pre}.v_proj.bias'])
     close_rel(np32(model.cross_kv[3, 0]).transpose(1, 0, 2).reshape(1500, 1280), k)
     close_rel(np32(model.cross_kv[3, 1]).transpose(1, 0, 2).reshape(1500, 1280), v)
+
+
+@pytest.mark.parametrize('n,offset', [(400, 0), (1120, 1), (16037, 3), (48000, 0), (48160, 1)])
+def test_log_mel_lengths_and_alignment(ext, hip_device, n, offset):
+    """Frame counts that leave partial frame blocks and finalize tiles (2, 7, 100, 300 and 301 frames, both
+    multiples of 4 and not) and waveforms and outputs that start off a 16-byte boundary, against the oracle."""
+    from flash_whisper_amd.audio import mel_filters
+    from oracle.logmel import log_mel
+
+    audio = (np.random.default_rng(n).standard_normal(n + offset) * 0.1).astype(np.float32)
+    frames = n // 160
+    filters = torch.from_numpy(mel_filters()).to(hip_device)
+    wave = torch.from_numpy(audio).to(hip_device)[offset:]
+    out = torch.empty(128 * frames + offset, device=hip_device)[offset:].view(128, frames)
+    out16 = torch.empty(frames, 128, dtype=torch.float16, device=hip_device)
+    ext.log_mel(wave, filters, out, out16, ext.log_mel_workspace(n))
+    got = out.cpu().numpy()
+    assert np.abs(got - log_mel(audio[offset:])).max() <= 1e-4
+    assert np.array_equal(out16.cpu().numpy(), got.T.astype(np.float16))

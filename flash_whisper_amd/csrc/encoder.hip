@@ -21,9 +21,10 @@ namespace {
 //  - Plain GEMMs (gemm_dma_kernel): global -> LDS copies into a ring of stages, operand fragments
 //    double-buffered in registers (see the pipeline notes above that kernel).
 //  - Implicit-GEMM conv: a 64-wide k stage of A row m is 64 contiguous channels of input row
-//    m * stride + tap - 1, so long-k convs use the same direct-to-LDS pipeline (padding rows copy
-//    from a zero row); short-k convs gather the A tile through registers (gemm_kernel: two staging
-//    sets, two LDS buffers).
+//    m * stride + tap - 1, so convs use the same direct-to-LDS pipeline (padding rows copy from a zero
+//    row).
+//  - Products of few rows: tiles of 32 x 32 to 96 x 64 whose k stages are dealt to the block's waves
+//    (gemm_ks_kernel); choose_tile picks the tile by the passes over the CUs and their cost.
 //  - Tile order: hardware deals blocks round-robin over the 8 XCDs; the block id is remapped so each
 //    XCD works on its own part of the tile grid and its L2 sees only that part's operand panels.
 // MFMA 32x32x16 f16 operand layout (lane l, g = l / 32):
@@ -71,9 +72,9 @@ struct GemmArgs {
 // b % 8), each with its own L2. With a grouping, XCD x owns one (ntm / xm) x (ntn / xn) rectangle of
 // the tile grid, so each XCD fetches only its slices of A and W. Otherwise each XCD takes a contiguous
 // run of row-major tiles (the tail beyond a multiple of 8 keeps its id). Both maps are bijective.
-template <int BM>
+template <int BM, int BN = kBN>
 __device__ __forceinline__ void tile_origin(const GemmArgs& g, int& m0, int& n0) {
-  const int ntn = g.n / kBN, ntm = (g.m + BM - 1) / BM;
+  const int ntn = g.n / BN, ntm = (g.m + BM - 1) / BM;
   const int bid = g.splits > 1 ? static_cast<int>(blockIdx.x) % (ntn * ntm) : static_cast<int>(blockIdx.x);
   int tm, tn;
   if (g.xm) {
@@ -87,7 +88,7 @@ __device__ __forceinline__ void tile_origin(const GemmArgs& g, int& m0, int& n0)
     tn = tile % ntn;
   }
   m0 = tm * BM;
-  n0 = tn * kBN;
+  n0 = tn * BN;
 }
 
 constexpr bool epi_reads_res(int epi) {
@@ -155,74 +156,6 @@ __device__ __forceinline__ float epilogue_value(int epi, float acc, float b, con
 }
 
 
-template <int BM>
-struct GemmStage {
-  static constexpr int kA = BM * 8 / 256;   // 16-byte A chunks per thread per stage
-  static constexpr int kB = kBN * 8 / 256;  // 16-byte B chunks per thread per stage
-  u32x4 a[kA];
-  u32x4 b[kB];
-};
-
-template <int BM, bool CONV>
-__device__ __forceinline__ void gemm_load(const GemmArgs& g, int m0, int n0, int k0, int tid, GemmStage<BM>& st) {
-#pragma unroll
-  for (int i = 0; i < GemmStage<BM>::kA; ++i) {
-    const int c = tid + 256 * i;
-    const int row = c >> 3, kc = (c & 7) * 8;
-    const int gm = m0 + row;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (gm < g.m) {
-      if constexpr (CONV) {
-        const int kk = k0 + kc;
-        const int tap = kk / g.c_in, ch = kk - tap * g.c_in;
-        const int src = gm * g.conv_stride + tap - 1;
-        if (src >= 0 && src < g.t_in) v = *reinterpret_cast<const u32x4*>(g.a + static_cast<size_t>(src) * g.c_in + ch);
-      } else {
-        v = *reinterpret_cast<const u32x4*>(g.a + static_cast<size_t>(gm) * g.lda + k0 + kc);
-      }
-    }
-    st.a[i] = v;
-  }
-#pragma unroll
-  for (int i = 0; i < GemmStage<BM>::kB; ++i) {
-    const int c = tid + 256 * i;
-    const int row = c >> 3, kc = (c & 7) * 8;
-    st.b[i] = *reinterpret_cast<const u32x4*>(g.w + static_cast<size_t>(n0 + row) * g.ldw + k0 + kc);
-  }
-}
-
-template <int BM>
-__device__ __forceinline__ void gemm_store(u32x4* As, u32x4* Bs, int tid, const GemmStage<BM>& st) {
-#pragma unroll
-  for (int i = 0; i < GemmStage<BM>::kA; ++i) {
-    const int c = tid + 256 * i;
-    As[swz(c >> 3, c & 7)] = st.a[i];
-  }
-#pragma unroll
-  for (int i = 0; i < GemmStage<BM>::kB; ++i) {
-    const int c = tid + 256 * i;
-    Bs[swz(c >> 3, c & 7)] = st.b[i];
-  }
-}
-
-template <int kTM, int kTN>
-__device__ __forceinline__ void gemm_mma(const u32x4* As, const u32x4* Bs, int wm, int wn, int lr, int lg,
-                                         f16v (&acc)[kTM][kTN]) {
-#pragma unroll
-  for (int s = 0; s < kBK / 16; ++s) {
-    h8v av[kTM], bv[kTN];
-#pragma unroll
-    for (int i = 0; i < kTM; ++i) av[i] = __builtin_bit_cast(h8v, As[swz(wm + 32 * i + lr, 2 * s + lg)]);
-#pragma unroll
-    for (int j = 0; j < kTN; ++j) bv[j] = __builtin_bit_cast(h8v, Bs[swz(wn + 32 * j + lr, 2 * s + lg)]);
-#pragma unroll
-    for (int i = 0; i < kTM; ++i)
-#pragma unroll
-      for (int j = 0; j < kTN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
-  }
-}
-
 // MFMA operand fragments of one 64-wide k stage for a wave: A rows wm + 32 i + lane % 32, B rows
 // wn + 32 j + lane % 32, k-step s covering k 16 s .. 16 s + 15.
 template <int kTM, int kTN>
@@ -288,8 +221,8 @@ __device__ __forceinline__ void mma_frags(const Frags<kTM, kTN>& f, f16v (&acc)[
 // The LDS ring depth ST is picked per tile height: 256-row tiles use three 48 KB stages (one 8-wave
 // block per CU); 128-row tiles (8 waves of 32 x 64; the split-k products) four 32 KB stages; 64-row
 // tiles (launched when 128-row tiles would leave CUs idle) four 24 KB stages (5 or 6 measured the same).
-// Tuning knobs (defaults measured on MI355X): ring depths per tile height, the minimum number of
-// 256-row tiles for that shape, waves per 256-row and 64-row block, and the XCD rectangle grouping.
+// Tuning knobs (defaults measured on MI355X): ring depths per tile height, waves per 256-row and 64-row
+// block, and the XCD rectangle grouping.
 // 8 waves on the 64-row tiles (two per SIMD) against 4: out projection 14.8 -> 14.35 us, stem conv
 // 36.0 -> 33.0 us (kernel trace, same box).
 #ifndef FW_ST128
@@ -304,9 +237,6 @@ __device__ __forceinline__ void mma_frags(const Frags<kTM, kTN>& f, f16v (&acc)[
 #ifndef FW_ST192
 #define FW_ST192 3
 #endif
-#ifndef FW_MIN_TILES256
-#define FW_MIN_TILES256 128
-#endif
 template <int BM>
 constexpr int dma_stages() {
   return BM == 256 ? FW_ST256 : BM == 192 ? FW_ST192 : BM == 128 ? FW_ST128 : FW_ST64;
@@ -317,7 +247,6 @@ template <int BM>
 constexpr bool ring_fits() { return dma_stages<BM>() >= 2 && dma_stages<BM>() * (BM + kBN) * 128 <= 160 * 1024; }
 static_assert(ring_fits<256>() && ring_fits<192>() && ring_fits<128>() && ring_fits<64>(),
               "FW_ST256 / FW_ST192 / FW_ST128 / FW_ST64: 2 or more stages within 160 KB of LDS");
-static_assert(FW_MIN_TILES256 >= 1, "FW_MIN_TILES256 must be positive");
 // Waves per block, in gemm_wave_cols columns (kBN / cols output columns each) and waves / cols rows;
 // each wave owns a (BM / rows) x (kBN / cols) tile. 192-row tiles use 2 x 4 waves of 96 x 32 and
 // 128-row tiles 4 x 2 waves of 32 x 64.
@@ -454,9 +383,9 @@ __device__ __forceinline__ void store_vt(const GemmArgs& g, const f16v (&acc)[kT
   }
 }
 
-template <int BM, int EPI, bool CONV = false>
+template <int BM, int EPI, bool CONV = false, int ST = dma_stages<BM>()>
 __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArgs g) {
-  constexpr int kDmaStages = dma_stages<BM>(), kNW = gemm_waves<BM>(), kNWN = gemm_wave_cols<BM>();
+  constexpr int kDmaStages = ST, kNW = gemm_waves<BM>(), kNWN = gemm_wave_cols<BM>();
   constexpr int kWM = BM / (kNW / kNWN), kTM = kWM / 32, kTN = kBN / kNWN / 32;
   static_assert(kWM % 32 == 0 && kTN >= 1 && BM % (8 * kNW) == 0, "wave tiling");
   constexpr int kStageBytes = (BM + kBN) * 128;
@@ -592,21 +521,79 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArg
   }
 }
 
-template <int BM, int EPI, bool CONV>
-__global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
-  constexpr int kWM = BM / 2;                // wave tile rows
-  constexpr int kTM = kWM / 32;              // MFMA tiles per wave along M
-  constexpr int kTN = 2;                     // MFMA tiles per wave along N (64 columns)
-  __shared__ __align__(16) u32x4 As0[BM * 8], As1[BM * 8];
-  __shared__ __align__(16) u32x4 Bs0[kBN * 8], Bs1[kBN * 8];
+// ---- k-sliced GEMM for few rows ----------------------------------------------------------------
+// out = epilogue(A W^T) where the tiles of gemm_dma_kernel would leave most CUs idle. A block's kKsWaves
+// waves all compute the whole TM x TN tile, wave w over the 64-wide k stages w, w + kKsWaves, ...: each
+// wave fills and reads a ring of its own, so the main loop has no barrier, and a stage's operands are
+// read from LDS once (waves that split the tile read the A or W half they share again: 64-row tiles of
+// 32 x 32 waves spend 512 LDS clocks a stage on 128 clocks of MFMA). The waves' sums are added in wave
+// order through LDS, then the epilogue runs on 4 adjacent columns a thread. What bounds it is the weights'
+// way from HBM: 128 KB or more in flight per CU. A 4-layer encoder over 251 frames, stem and cross K/V:
+// 424 -> 309 us (fc2 20.2 -> 13, out 10.7 -> 6.4 us a launch).
+constexpr int kKsWaves = 4;
+constexpr int kKsLds = 160 * 1024;
+template <int TM, int TN>
+constexpr int ks_stages() {  // ring depth per wave: what fits one block's LDS, at most 4
+  return kKsLds / (kKsWaves * (TM + TN) * 128) < 4 ? kKsLds / (kKsWaves * (TM + TN) * 128) : 4;
+}
+
+template <int TM, int TN, int EPI, bool CONV>
+__global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(GemmArgs g) {
+  constexpr int kST = ks_stages<TM, TN>(), kTM = TM / 32, kTN = TN / 32;
+  constexpr int kStageBytes = (TM + TN) * 128, kPer = (TM + TN) / 8;  // copies per stage
+  constexpr int kRowF = TN + 4;                                      // floats per staged row of sums
+  static_assert(kST >= 2 && (kST - 1) * kPer < 64, "ring depth");
+  static_assert(TM * kRowF * 4 <= kST * kStageBytes, "a wave's sums fit its ring");
+  __shared__ __align__(1024) u32x4 lds[kKsWaves * kST * kStageBytes / 16];
 
   int m0, n0;
-  tile_origin<BM>(g, m0, n0);
+  tile_origin<TM, TN>(g, m0, n0);
+  int split = 0;
+  if constexpr (EPI == kEpiPartial) {
+    split = static_cast<int>(blockIdx.x) / ((g.n / TN) * ((g.m + TM - 1) / TM));
+    g.a += static_cast<size_t>(split) * g.k;
+    g.w += static_cast<size_t>(split) * g.k;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lg = lane >> 5, rsub = lane >> 3, slot8 = lane & 7;
+  char* ring = reinterpret_cast<char*>(lds) + wave * (kST * kStageBytes);
+  const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * kWM, wn = (wave & 1) * 64;
-  const int lr = lane & 31, lg = lane >> 5;
-
+  // byte offsets of this lane's chunk of every copy of a stage (A rows, then W rows)
+  uint32_t aoff[TM / 8], woff[TN / 8];
+  if constexpr (!CONV) {
+#pragma unroll
+    for (int i = 0; i < TM / 8; ++i) {
+      const int row = i * 8 + rsub;
+      aoff[i] = static_cast<uint32_t>((static_cast<size_t>(min(m0 + row, g.m - 1)) * g.lda + swz_slot(row, slot8) * 8) * 2);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TN / 8; ++i) {
+    const int row = i * 8 + rsub;
+    woff[i] = static_cast<uint32_t>((static_cast<size_t>(n0 + row) * g.ldw + swz_slot(row, slot8) * 8) * 2);
+  }
+  auto issue = [&](int kt, int slot) {
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(ring0 + slot * kStageBytes);
+    const size_t kb = static_cast<size_t>(kt) * (kBK * 2);
+    if constexpr (CONV) {
+      const int tap = kt * kBK / g.c_in, ch0 = kt * kBK - tap * g.c_in;
+#pragma unroll
+      for (int i = 0; i < TM / 8; ++i) {
+        const int row = i * 8 + rsub;
+        const int r = min(m0 + row, g.m - 1) * g.conv_stride + tap - 1;
+        const _Float16* src = (r >= 0 && r < g.t_in) ? g.a + static_cast<size_t>(r) * g.c_in + ch0 : g_zero_row;
+        dma16(src + swz_slot(row, slot8) * 8, dst + i * 1024);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TM / 8; ++i) dma16_s(aoff[i], reinterpret_cast<const char*>(g.a) + kb, dst + i * 1024);
+    }
+#pragma unroll
+    for (int i = 0; i < TN / 8; ++i)
+      dma16_s(woff[i], reinterpret_cast<const char*>(g.w) + kb, dst + TM * 128 + i * 1024);
+  };
+  const FragOffsets fo = frag_offsets<TM>(0, 0, lr, lg);
   f16v acc[kTM][kTN];
 #pragma unroll
   for (int i = 0; i < kTM; ++i)
@@ -615,46 +602,100 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  GemmStage<BM> st0, st1;
-  const int kt_n = g.k / kBK;
-  gemm_load<BM, CONV>(g, m0, n0, 0, tid, st0);
-  gemm_store<BM>(As0, Bs0, tid, st0);
-  if (kt_n > 1) gemm_load<BM, CONV>(g, m0, n0, kBK, tid, st1);
-  __syncthreads();
-  for (int kt = 0; kt < kt_n; kt += 2) {
-    // stage kt in LDS buffer 0; stage kt + 1 arriving in st1
-    if (kt + 2 < kt_n) gemm_load<BM, CONV>(g, m0, n0, (kt + 2) * kBK, tid, st0);
-    gemm_mma<kTM, kTN>(As0, Bs0, wm, wn, lr, lg, acc);
-    if (kt + 1 < kt_n) gemm_store<BM>(As1, Bs1, tid, st1);
-    lds_barrier();
-    if (kt + 1 >= kt_n) break;
-    // stage kt + 1 in LDS buffer 1; stage kt + 2 arriving in st0
-    if (kt + 3 < kt_n) gemm_load<BM, CONV>(g, m0, n0, (kt + 3) * kBK, tid, st1);
-    gemm_mma<kTM, kTN>(As1, Bs1, wm, wn, lr, lg, acc);
-    if (kt + 2 < kt_n) gemm_store<BM>(As0, Bs0, tid, st0);
-    lds_barrier();
+  const int kt_all = g.k / kBK, n_st = (kt_all - wave + kKsWaves - 1) / kKsWaves;  // this wave's stages
+#pragma unroll
+  for (int s = 0; s < kST; ++s)
+    if (s < n_st) issue(wave + s * kKsWaves, s);
+  if (n_st > 0) {
+    Frags<kTM, kTN> fa, fb;
+    wait_stages_ahead<kPer, kST - 1>(min(kST - 1, n_st - 1));
+    load_frags<kTM, kTN>(ring, fo, fa);
+    int cur = 0;
+    auto step = [&](int i, const Frags<kTM, kTN>& now, Frags<kTM, kTN>& nxt) {
+      wait_stages_ahead<kPer, kST - 1>(min(kST - 2, n_st - 2 - i));
+      lds_reads_done();  // stage i is in registers: its slot is free
+      if (i + kST < n_st) issue(wave + (i + kST) * kKsWaves, cur);
+      cur = cur + 1 == kST ? 0 : cur + 1;
+      load_frags<kTM, kTN>(ring + cur * kStageBytes, fo, nxt);
+      mma_frags<kTM, kTN, true>(now, acc);
+    };
+    int i = 0;
+    for (; i + 2 < n_st; i += 2) {
+      step(i, fa, fb);
+      step(i + 1, fb, fa);
+    }
+    if (i + 1 < n_st) {
+      step(i, fa, fb);
+      mma_frags<kTM, kTN, true>(fb, acc);
+    } else {
+      mma_frags<kTM, kTN, true>(fa, acc);
+    }
   }
-
+  // this wave's sums, row by row, into its own ring (every copy has landed and been read)
+  lds_reads_done();
+  float* sums = reinterpret_cast<float*>(ring);
 #pragma unroll
-  for (int j = 0; j < kTN; ++j) {
-    const int col = n0 + wn + 32 * j + lr;
-    const float b = g.bias ? h2f(g.bias[col]) : 0.f;
+  for (int i = 0; i < kTM; ++i)
 #pragma unroll
-    for (int i = 0; i < kTM; ++i) {
+    for (int j = 0; j < kTN; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
-        if (row < g.m) {
-          if constexpr (EPI == kEpiCrossKV) {
-            // col = ((layer * 2 + kv) * heads + head) * 64 + d
-            const int d = col & 63, lhk = col >> 6;
-            const size_t o = (static_cast<size_t>(lhk) * g.t_len + row) * 64 + d;
-            g.out[o] = f2h(acc[i][j][r] + b);
-          } else {
-            g.out[static_cast<size_t>(row) * g.ldo + col] = f2h(epilogue_value(EPI, acc[i][j][r], b, g, row, col));
-          }
-        }
+      for (int rq = 0; rq < 4; ++rq) {
+        f4v v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * rq + e];
+        *reinterpret_cast<f4v*>(sums + (32 * i + lr) * kRowF + 32 * j + 8 * rq + 4 * lg) = v;
       }
+  __syncthreads();
+  const float* part0 = reinterpret_cast<const float*>(lds);
+  constexpr int kWaveF = kST * kStageBytes / 4;  // floats between the waves' sums
+  if constexpr (EPI == kEpiQkvVt) {
+    if (n0 >= 2 * g.q_cols) {  // a tile of v columns: 4 adjacent keys of one column per thread, stored transposed
+      _Float16* dst = g.vt + static_cast<size_t>(n0 - 2 * g.q_cols) * g.vt_pad;
+      for (int c = tid; c < TM / 4 * TN; c += kKsWaves * 64) {
+        const int col = c / (TM / 4), rl = c % (TM / 4) * 4;  // rows rl .. rl + 3 stay adjacent under vt_pos
+        const float b = g.bias ? h2f(g.bias[n0 + col]) : 0.f;
+        h4v o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float v = 0.f;
+#pragma unroll
+          for (int w = 0; w < kKsWaves; ++w) v += part0[w * kWaveF + (rl + e) * kRowF + col];
+          o[e] = m0 + rl + e < g.m ? f2h(v + b) : static_cast<_Float16>(0.f);
+        }
+        if (m0 + rl < g.vt_pad) *reinterpret_cast<h4v*>(dst + static_cast<size_t>(col) * g.vt_pad + m0 + vt_pos(rl)) = o;
+      }
+      // the last row tile may end before V^T's padding to whole 64-key tiles: zeros from there on
+      const int pad4 = m0 + TM >= g.m ? (g.vt_pad - m0 - TM) / 4 : 0;
+      for (int c = tid; c < pad4 * TN; c += kKsWaves * 64)
+        *reinterpret_cast<h4v*>(dst + static_cast<size_t>(c / pad4) * g.vt_pad + m0 + TM + c % pad4 * 4) = h4v{};
+      return;
+    }
+  }
+  constexpr int kCols4 = TN / 4;
+#pragma unroll
+  for (int c = tid; c < TM * kCols4; c += kKsWaves * 64) {
+    const int rl = c / kCols4, cl = c % kCols4 * 4, row = m0 + rl, col = n0 + cl;
+    f4v v = *reinterpret_cast<const f4v*>(part0 + rl * kRowF + cl);
+#pragma unroll
+    for (int w = 1; w < kKsWaves; ++w) {
+      const f4v u = *reinterpret_cast<const f4v*>(part0 + w * kWaveF + rl * kRowF + cl);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += u[e];
+    }
+    if (row >= g.m) continue;
+    if constexpr (EPI == kEpiPartial) {
+      *reinterpret_cast<f4v*>(g.part + (static_cast<size_t>(split) * g.m + row) * g.n + col) = v;
+    } else {
+      h4v bb = {}, rv = {}, o;
+      if (g.bias) bb = *reinterpret_cast<const h4v*>(g.bias + col);
+      if constexpr (epi_reads_res(EPI)) rv = *reinterpret_cast<const h4v*>(g.res + static_cast<size_t>(row) * g.ldr + col);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = f2h(epilogue_apply(EPI, v[e], h2f(bb[e]), h2f(rv[e]), col + e, g.q_cols));
+      if constexpr (EPI == kEpiCrossKV)
+        *reinterpret_cast<h4v*>(g.out + (static_cast<size_t>(col >> 6) * g.t_len + row) * 64 + (col & 63)) = o;
+      else
+        *reinterpret_cast<h4v*>(g.out + static_cast<size_t>(row) * g.ldo + col) = o;
     }
   }
 }
@@ -665,10 +706,10 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
 static_assert(FW_XCD_GROUP == 0 || FW_XCD_GROUP == 1, "FW_XCD_GROUP is a switch (0 or 1)");
 // Picks the XCD rectangle grid that divides the tile grid and moves the fewest bytes into the L2s:
 // A is fetched once per column group (xn), W once per row group (xm).
-void choose_xcd_groups(GemmArgs& g, int bm) {
+void choose_xcd_groups(GemmArgs& g, int bm, int bn = kBN) {
   g.xm = g.xn = 0;
   if (!FW_XCD_GROUP || g.conv_stride) return;
-  const int ntm = (g.m + bm - 1) / bm, ntn = g.n / kBN;
+  const int ntm = (g.m + bm - 1) / bm, ntn = g.n / bn;
   double best = 0;
   for (int xm = 1; xm <= 8; xm *= 2) {
     const int xn = 8 / xm;
@@ -690,84 +731,131 @@ bool copy_offsets_fit(const GemmArgs& g) {
          (static_cast<size_t>(g.n - 1) * g.ldw + kBK) * 2 < kLimit;
 }
 
-template <int BM>
-int launch_gemm_bm(GemmArgs g, int epi, hipStream_t s) {
-  const int tiles = (g.n / kBN) * ((g.m + BM - 1) / BM);
-  const dim3 grid(tiles);
+template <int BM, bool CONV, int ST = dma_stages<BM>()>
+int launch_dma(GemmArgs g, int epi, hipStream_t s) {
+  const dim3 grid((g.n / kBN) * ((g.m + BM - 1) / BM)), block(gemm_waves<BM>() * 64);
   choose_xcd_groups(g, BM);
-  // Implicit convs with a long k (the stride-2 1280 -> 1280 stem conv, k = 3840) use the direct-to-LDS
-  // pipeline (75 -> 37 us); with a short k (the 128 -> 1280 conv, k = 384: six stages) the ring's
-  // fill and drain dominate and the register-staged kernel, whose small LDS footprint keeps two
-  // blocks per CU, is faster (15 us against 18-19 us).
-  if (g.conv_stride && g.k >= 1024) {
-    switch (epi) {
-#define FW_CONV_CASE(E) \
-  case E:               \
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, E, true>), grid, dim3(gemm_waves<BM>() * 64), 0, s, g); break;
-      FW_CONV_CASE(FW_EPI_BIAS)
-      FW_CONV_CASE(FW_EPI_BIAS_GELU)
-      FW_CONV_CASE(FW_EPI_BIAS_GELU_POS)
-#undef FW_CONV_CASE
-      default:
-        return fw_fail(FW_EINVAL, "conv1d: unsupported epilogue %d", epi);
-    }
-    return fw_check_launch("conv1d");
-  }
-  if constexpr (BM <= 128) {
-  if (g.conv_stride) {
-    switch (epi) {
-      case FW_EPI_BIAS: hipLaunchKernelGGL((gemm_kernel<BM, FW_EPI_BIAS, true>), grid, dim3(256), 0, s, g); break;
-      case FW_EPI_BIAS_GELU:
-        hipLaunchKernelGGL((gemm_kernel<BM, FW_EPI_BIAS_GELU, true>), grid, dim3(256), 0, s, g);
-        break;
-      case FW_EPI_BIAS_GELU_POS:
-        hipLaunchKernelGGL((gemm_kernel<BM, FW_EPI_BIAS_GELU_POS, true>), grid, dim3(256), 0, s, g);
-        break;
-      default:
-        return fw_fail(FW_EINVAL, "conv1d: unsupported epilogue %d", epi);
-    }
-    return fw_check_launch("conv1d");
-  }
-  }
-  if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
   switch (epi) {
-#define FW_GEMM_CASE(E) \
-  case E:               \
-    hipLaunchKernelGGL((gemm_dma_kernel<BM, E>), grid, dim3(gemm_waves<BM>() * 64), 0, s, g); break;
-    FW_GEMM_CASE(FW_EPI_BIAS)
-    FW_GEMM_CASE(FW_EPI_BIAS_GELU)
-    FW_GEMM_CASE(FW_EPI_BIAS_RESID)
-    FW_GEMM_CASE(FW_EPI_BIAS_RESID_CLAMP)
-    FW_GEMM_CASE(FW_EPI_BIAS_GELU_POS)
-    FW_GEMM_CASE(FW_EPI_SCALE_Q)
-    FW_GEMM_CASE(kEpiCrossKV)
-    FW_GEMM_CASE(kEpiQkvVt)
+#define FW_GEMM_CASE(E, C) \
+  case E:                  \
+    if constexpr (C || !CONV) hipLaunchKernelGGL((gemm_dma_kernel<BM, E, CONV, ST>), grid, block, 0, s, g); \
+    break;
+    FW_GEMM_CASE(FW_EPI_BIAS, true)
+    FW_GEMM_CASE(FW_EPI_BIAS_GELU, true)
+    FW_GEMM_CASE(FW_EPI_BIAS_GELU_POS, true)
+    FW_GEMM_CASE(FW_EPI_BIAS_RESID, false)
+    FW_GEMM_CASE(FW_EPI_BIAS_RESID_CLAMP, false)
+    FW_GEMM_CASE(FW_EPI_SCALE_Q, false)
+    FW_GEMM_CASE(kEpiCrossKV, false)
+    FW_GEMM_CASE(kEpiQkvVt, false)
 #undef FW_GEMM_CASE
     default:
       return fw_fail(FW_EINVAL, "gemm: unknown epilogue %d", epi);
   }
-  return fw_check_launch("gemm");
+  return fw_check_launch(CONV ? "conv1d" : "gemm");
 }
 
-// 256-row tiles (8 waves, 48 KB stages) when they still cover half the CUs: they do twice the MFMA
-// work per byte staged of 128-row tiles. When 256-row tiles would leave a quarter of the CUs idle and
-// 192-row tiles still fit in one pass (q/k/v: 180 -> 240 tiles), 192-row tiles: each SIMD then does
-// 3/4 of the MFMA work and each CU stages 5/6 of the bytes (4.90 -> 4.78 ms per encoder on MI355X).
-// Fewer 128-row tiles than CUs leaves the chip idle: use 64-row tiles then. The implicit-GEMM conv
-// stays on the register-staged kernel (<= 128 rows).
-#ifndef FW_USE192
-#define FW_USE192 1
-#endif
-static_assert(FW_USE192 == 0 || FW_USE192 == 1, "FW_USE192 is a switch (0 or 1)");
+template <int TM, int TN, bool CONV>
+int launch_ks(GemmArgs g, int epi, hipStream_t s) {
+  const int tiles = (g.n / TN) * ((g.m + TM - 1) / TM);
+  const dim3 grid(tiles * (g.splits > 1 ? g.splits : 1)), block(kKsWaves * 64);
+  choose_xcd_groups(g, TM, TN);
+  switch (epi) {
+#define FW_KS_CASE(E, C) \
+  case E:                \
+    if constexpr (C) hipLaunchKernelGGL((gemm_ks_kernel<TM, TN, E, CONV>), grid, block, 0, s, g); \
+    break;
+    FW_KS_CASE(FW_EPI_BIAS, true)
+    FW_KS_CASE(FW_EPI_BIAS_GELU, true)
+    FW_KS_CASE(FW_EPI_BIAS_GELU_POS, true)
+    FW_KS_CASE(FW_EPI_BIAS_RESID, !CONV)
+    FW_KS_CASE(FW_EPI_BIAS_RESID_CLAMP, !CONV)
+    FW_KS_CASE(FW_EPI_SCALE_Q, !CONV)
+    FW_KS_CASE(kEpiCrossKV, !CONV)
+    FW_KS_CASE(kEpiQkvVt, !CONV)
+    FW_KS_CASE(kEpiPartial, !CONV)
+#undef FW_KS_CASE
+    default:
+      return fw_fail(FW_EINVAL, "gemm: unknown epilogue %d", epi);
+  }
+  return fw_check_launch(CONV ? "conv1d" : "gemm");
+}
+
+// The tile: the fewest passes over the CUs (one block per CU: each tile's ring takes most of its LDS) at
+// the tile's cost, kPassUs + k stages x per_stage. Both are fits to times on MI355X with weights cold (a
+// graph over >300 MB of them; m = 50 .. 1500, n = 1280, 3840, 5120, k = 1280, 2 x 2560 and the convs'
+// 3840), good to about 20%; what decides is mostly the passes. Measured us for (m, n, k) by tile:
+//   (50, 1280, 1280)   32x32 4.8, 64x32 6.2, 64x64 7.8, 64x128 9.6
+//   (251, 1280, 1280)  32x32 7.8 (2 passes), 64x32 6.3, 64x64 8.2, 64x128 10.5, 128x128 15.1
+//   (251, 5120, 1280)  64x64 19.6 (2), 96x64 13.6, 64x128 14.4, 128x128 18.7
+//   (640, 5120, 1280)  64x128 26 (2), 128x128 19.0, 192x128 21.9, 256x128 26.2
+//   (1000, 3840, 1280) 64x128 24.2 (2), 128x128 18.1, 192x128 19.6, 256x128 24.6
+//   (1200, 5120, 1280) 128x128 34.3 (2), 192x128 38.0 (2), 256x128 30.4
+//   (251, 1280, 2 x 2560) 64x32 19.4 (2), 64x64 15.1, 96x64 17.7, 128x128 28.4
+//   (400, 1280, 2 x 2560) 64x64 26.1 (2), 96x64 17.6, 128x128 23.1
+enum Tile { kD256, kD192, kD128, kD64, kS96x64, kS64x64, kS64x32, kS32x32, kTiles };
+struct TileCost {
+  int rows, cols;
+  float per_stage;  // us per 64-wide k stage and pass
+};
+constexpr TileCost kTileCost[kTiles] = {{256, 128, 1.15f}, {192, 128, 0.85f}, {128, 128, 0.62f}, {64, 128, 0.42f},
+                                        {96, 64, 0.40f},   {64, 64, 0.28f},   {64, 32, 0.18f},   {32, 32, 0.11f}};
+constexpr float kPassUs = 4.f;
+constexpr int kCus = 256;
+
+template <class Allowed>
+Tile choose_tile(const GemmArgs& g, Allowed allowed) {
+  Tile best = kD128;
+  float best_us = 0.f;
+  for (int t = 0; t < kTiles; ++t) {
+    if (!allowed(static_cast<Tile>(t))) continue;
+    const TileCost& c = kTileCost[t];
+    const int64_t blocks = static_cast<int64_t>(g.n / c.cols) * ((g.m + c.rows - 1) / c.rows) * (g.splits > 1 ? g.splits : 1);
+    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * c.per_stage);
+    if (best_us == 0.f || us < best_us) {
+      best = static_cast<Tile>(t);
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+// The sliced kernel's and the 64-row tiles' epilogues move 4 adjacent columns at a time.
+bool vector_epilogue(const GemmArgs& g) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.out) | reinterpret_cast<uintptr_t>(g.res);
+  return !(p & 7u);
+}
+
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
-  const int tiles256 = (g.n / kBN) * ((g.m + 255) / 256);
-  const int tiles192 = (g.n / kBN) * ((g.m + 191) / 192);
-  const int tiles128 = (g.n / kBN) * ((g.m + 127) / 128);
-  if (FW_USE192 && !g.conv_stride && tiles256 < 192 && tiles256 >= FW_MIN_TILES256 && tiles192 <= 256)
-    return launch_gemm_bm<192>(g, epi, s);
-  if (!g.conv_stride && tiles256 >= FW_MIN_TILES256) return launch_gemm_bm<256>(g, epi, s);
-  if (tiles128 < 256) return launch_gemm_bm<64>(g, epi, s);
-  return launch_gemm_bm<128>(g, epi, s);
+  if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
+  const bool vec = vector_epilogue(g), qkv = epi == kEpiQkvVt;
+  // (the 64-row tiles store q/k/v by element, so they need no alignment there)
+  switch (choose_tile(g, [&](Tile t) { return vec || t < kD64 || (qkv && t == kD64); })) {
+    case kD256: return launch_dma<256, false>(g, epi, s);
+    case kD192: return launch_dma<192, false>(g, epi, s);
+    case kD64: return launch_dma<64, false>(g, epi, s);
+    case kS96x64: return launch_ks<96, 64, false>(g, epi, s);
+    case kS64x64: return launch_ks<64, 64, false>(g, epi, s);
+    case kS64x32: return launch_ks<64, 32, false>(g, epi, s);
+    case kS32x32: return launch_ks<32, 32, false>(g, epi, s);
+    default: return launch_dma<128, false>(g, epi, s);
+  }
+}
+
+// Convs. With a short k (the 128 -> 1280 conv of the stem, k = 384: six stages) a pass is mostly fill,
+// drain and epilogue: past one pass of 64 x 64 tiles, 64-row tiles with a 3-deep ring, two blocks on a
+// CU, so that one's epilogue runs beside the other's copies (3000 rows: 9.9 us against 12.6 for a
+// register-staged gather, 10.3 for a 2-deep ring and 10.1 for 128-row tiles; 1000 rows: 6.7, 10.5, 7.8, 9.4).
+int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
+  const bool vec = vector_epilogue(g) && copy_offsets_fit(g);  // (the sliced kernel's weight offsets are 32-bit)
+  const Tile t = choose_tile(g, [&](Tile c) { return c == kD128 || (vec && c >= kD64); });
+  if (t == kS64x64) return launch_ks<64, 64, true>(g, epi, s);
+  if (t == kS64x32) return launch_ks<64, 32, true>(g, epi, s);
+  if (t == kS32x32) return launch_ks<32, 32, true>(g, epi, s);
+  if (vec && g.k < 1024) return launch_dma<64, true, 3>(g, epi, s);
+  if (t == kS96x64) return launch_ks<96, 64, true>(g, epi, s);
+  if (t == kD64) return launch_dma<64, true>(g, epi, s);
+  return launch_dma<128, true>(g, epi, s);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -950,7 +1038,7 @@ extern "C" int fw_conv1d(const void* x, int t_in, int c_in, int stride, const vo
   GemmArgs g{static_cast<const _Float16*>(x), c_in, static_cast<const _Float16*>(wp), 3 * c_in,
              static_cast<const _Float16*>(bias), static_cast<_Float16*>(out), c_out,
              static_cast<const _Float16*>(res), c_out, t_out, c_out, 3 * c_in, 0, stride, t_in, c_in, 0, 0};
-  return launch_gemm(g, epilogue, stream);
+  return launch_conv(g, epilogue, stream);
 }
 
 extern "C" int fw_layernorm_rows(const void* x, const void* gamma, const void* beta, void* y, int rows, int n,
@@ -984,10 +1072,17 @@ extern "C" int fw_gemm_splitk(const void* a, int lda, const void* w, int ldw, fl
   g.k = k / splits;  // per split
   g.splits = splits;
   g.part = part;
+  if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm_splitk: each operand must span less than 4 GiB");
+  switch (choose_tile(g, [](Tile t) { return t == kD128 || t > kD64; })) {
+    case kS96x64: return launch_ks<96, 64, false>(g, kEpiPartial, stream);
+    case kS64x64: return launch_ks<64, 64, false>(g, kEpiPartial, stream);
+    case kS64x32: return launch_ks<64, 32, false>(g, kEpiPartial, stream);
+    case kS32x32: return launch_ks<32, 32, false>(g, kEpiPartial, stream);
+    default: break;
+  }
   // the XCD rectangles of the plain GEMMs (both k halves of a tile land on the same XCD when the tile
   // count is a multiple of 8): 126 -> 84 MB fetched from beyond L2 for the encoder's fc2
   choose_xcd_groups(g, 128);
-  if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm_splitk: each operand must span less than 4 GiB");
   const int tiles = (n / kBN) * ((m + 127) / 128);
   hipLaunchKernelGGL((gemm_dma_kernel<128, kEpiPartial>), dim3(splits * tiles), dim3(gemm_waves<128>() * 64), 0,
                      stream, g);

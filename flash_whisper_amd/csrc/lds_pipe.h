@@ -68,6 +68,12 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_barrier" ::: "memory");
 }
 
+// Waits for this wave's own LDS accesses; no LDS access or copy moves across it.
+__device__ __forceinline__ void lds_reads_done() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("" ::: "memory");
+}
+
 // Keys per transposed-V row: seq rounded up to whole 64-key attention tiles.
 __host__ __device__ constexpr int vt_pad(int seq) { return (seq + 63) / 64 * 64; }
 

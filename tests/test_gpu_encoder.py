@@ -65,6 +65,27 @@ def test_gemm_epilogues(ext, hip_device, m, n, k, epi):
     close_rel(np32(out), ref, scale=scale)
 
 
+# few rows: the sliced tiles (32 x 32, 64 x 32, 64 x 64 and 96 x 64 in turn), fewer k stages than waves, a
+# count of stages that does not divide by the waves, and partial last row tiles
+@pytest.mark.parametrize('m,n,k,epi', [(1, 128, 64, 0), (33, 1280, 64, 4), (50, 1280, 1280, 2), (97, 1280, 192, 3),
+                                       (251, 1280, 1280, 2), (129, 3840, 1280, 5), (251, 5120, 1280, 1)])
+def test_gemm_few_rows(ext, hip_device, m, n, k, epi):
+    test_gemm_epilogues(ext, hip_device, m, n, k, epi)
+
+
+@pytest.mark.parametrize('m', [1, 64, 65, 251, 400, 577])
+def test_gemm_splitk_few_rows(ext, hip_device, m):
+    """Both k halves of fc2 by the sliced tiles (and 128-row tiles at 577), each against its own product."""
+    dev = hip_device
+    rng = np.random.default_rng(m)
+    a, w = np.float16(0.5 * rng.standard_normal((m, 5120))), np.float16(0.02 * rng.standard_normal((1280, 5120)))
+    part = torch.full((2, m, 1280), float('nan'), dtype=torch.float32, device=dev)
+    ext.gemm_splitk(h16(a, dev), h16(w, dev), part)
+    for half in range(2):
+        c = slice(2560 * half, 2560 * half + 2560)
+        close_rel(np32(part[half]), a[:, c].astype(np.float64) @ w[:, c].astype(np.float64).T, rtol=1e-4)
+
+
 def _f16_order(v):
     """fp16 values -> integers in value order (adjacent fp16 numbers differ by 1)."""
     bits = np.asarray(v, np.float16).view(np.int16).astype(np.int32)
@@ -155,7 +176,8 @@ def test_gemm_row_strided_views(ext, hip_device):
     assert float(out_big[:, :128].abs().max()) == 0 and float(out_big[:, 256:].abs().max()) == 0
 
 
-@pytest.mark.parametrize('stride,c_in,t_in', [(1, 128, 3000), (2, 1280, 3000), (2, 128, 61)])
+@pytest.mark.parametrize('stride,c_in,t_in', [(1, 128, 3000), (2, 1280, 3000), (2, 128, 61), (1, 128, 1001), (1, 128, 502),
+                                              (1, 64, 1), (2, 1280, 99), (2, 1280, 502), (2, 1280, 1281)])
 def test_conv1d(ext, hip_device, stride, c_in, t_in):
     dev = hip_device
     rng = np.random.default_rng(stride + c_in)
@@ -217,7 +239,7 @@ def test_encoder_attention(ext, hip_device, seq, heads, qscale):
     close_rel(np32(out), _attn_ref(qkv, heads))
 
 
-@pytest.mark.parametrize('m', [1500, 77, 1])
+@pytest.mark.parametrize('m', [1500, 77, 1, 65, 97, 130, 251])
 def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m):
     """The fused q/k/v projection writes the FW_EPI_SCALE_Q GEMM's q and k columns and, for v, exactly
     what fw_encoder_pack_vt makes of that GEMM's v columns (padding keys zero)."""

@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArg
 // 32 x 32 waves spend 512 LDS clocks a stage on 128 clocks of MFMA). The waves' sums are added in wave
 // order through LDS, then the epilogue runs on 4 adjacent columns a thread. What bounds it is the weights'
 // way from HBM: 128 KB or more in flight per CU. A 4-layer encoder over 251 frames, stem and cross K/V:
-// 424 -> 309 us (fc2 20.2 -> 13, out 10.7 -> 6.4 us a launch).
+// 424 -> 309 us (fc2 20.2 -> 12.3, out 10.7 -> 6.7 us a launch).
 constexpr int kKsWaves = 4;
 constexpr int kKsLds = 160 * 1024;
 template <int TM, int TN>

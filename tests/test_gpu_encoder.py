@@ -222,7 +222,8 @@ def _attn_ref(qkv, heads):
 
 
 @pytest.mark.parametrize('seq,heads,qscale', [(1500, 20, 0.125), (100, 2, 0.125), (1500, 20, 0.6), (33, 1, 0.3),
-                                               (1496, 3, 0.2), (1, 2, 0.125), (64, 1, 0.5), (129, 2, 0.125)])
+                                               (1496, 3, 0.2), (1, 2, 0.125), (64, 1, 0.5), (129, 2, 0.125),
+                                               (128, 2, 0.3), (193, 2, 0.3), (256, 1, 0.3), (321, 3, 0.3), (833, 20, 0.2)])
 def test_encoder_attention(ext, hip_device, seq, heads, qscale):
     dev = hip_device
     rng = np.random.default_rng(seq + heads)

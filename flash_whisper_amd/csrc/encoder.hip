@@ -787,7 +787,8 @@ int launch_ks(GemmArgs g, int epi, hipStream_t s) {
 // 3840), good to about 20%; what decides is mostly the passes. Measured us for (m, n, k) by tile:
 //   (50, 1280, 1280)   32x32 4.8, 64x32 6.2, 64x64 7.8, 64x128 9.6
 //   (251, 1280, 1280)  32x32 7.8 (2 passes), 64x32 6.3, 64x64 8.2, 64x128 10.5, 128x128 15.1
-//   (251, 5120, 1280)  64x64 19.6 (2), 96x64 13.6, 64x128 14.4, 128x128 18.7
+//   (251, 5120, 1280)  64x64 19.6 (2), 96x64 14.0, 64x128 14.4, 128x128 18.7 (weights in L2: 96x64 11.3, 64x128 9.9)
+//   (1000, 1280, 1280) 96x64 12.8, 64x128 10.7
 //   (640, 5120, 1280)  64x128 26 (2), 128x128 19.0, 192x128 21.9, 256x128 26.2
 //   (1000, 3840, 1280) 64x128 24.2 (2), 128x128 18.1, 192x128 19.6, 256x128 24.6
 //   (1200, 5120, 1280) 128x128 34.3 (2), 192x128 38.0 (2), 256x128 30.4
@@ -799,7 +800,7 @@ struct TileCost {
   float per_stage;  // us per 64-wide k stage and pass
 };
 constexpr TileCost kTileCost[kTiles] = {{256, 128, 1.15f}, {192, 128, 0.85f}, {128, 128, 0.62f}, {64, 128, 0.42f},
-                                        {96, 64, 0.40f},   {64, 64, 0.28f},   {64, 32, 0.18f},   {32, 32, 0.11f}};
+                                        {96, 64, 0.43f},   {64, 64, 0.28f},   {64, 32, 0.18f},   {32, 32, 0.11f}};
 constexpr float kPassUs = 4.f;
 constexpr int kCus = 256;
 
@@ -811,7 +812,9 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
     if (!allowed(static_cast<Tile>(t))) continue;
     const TileCost& c = kTileCost[t];
     const int64_t blocks = static_cast<int64_t>(g.n / c.cols) * ((g.m + c.rows - 1) / c.rows) * (g.splits > 1 ? g.splits : 1);
-    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * c.per_stage);
+    // the direct-to-LDS kernel works out a conv's source rows for every copy
+    const float stage = g.conv_stride && t <= kD64 ? 1.1f * c.per_stage : c.per_stage;
+    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * stage);
     if (best_us == 0.f || us < best_us) {
       best = static_cast<Tile>(t);
       best_us = us;

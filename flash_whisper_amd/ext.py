@@ -28,8 +28,13 @@ MAX_BATCH = 4  # decoder positions per batched launch (the prompt)
 WAVE_CHUNK = 240000  # samples per staged chunk of the waveform upload (half of 30 s: smaller chunks measured slower)
 
 
+_F16, _F32, _I64 = torch.float16, torch.float32, torch.int64
+_device, _raw_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+
+
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream's handle, without the Stream object torch.cuda.current_stream() makes (1 us)."""
+    return _raw_stream(_device())
 
 
 def _ptr(t):
@@ -39,6 +44,20 @@ def _ptr(t):
 def _require(cond, msg):
     if not cond:
         raise RuntimeError(msg)
+
+
+# A call of an op is a few microseconds of kernels, so the checks of a valid call go through these two
+# (about 0.3 us a tensor); only a call they refuse runs the named checks below, which say what is wrong.
+def _all_contiguous(dtype, *tensors):
+    """Whether every argument is a contiguous CUDA tensor of `dtype`."""
+    for t in tensors:
+        if not isinstance(t, torch.Tensor) or t.dtype is not dtype or not t.is_cuda or not t.is_contiguous():
+            return False
+    return True
+
+
+def _halves(*tensors):
+    return _all_contiguous(_F16, *tensors)
 
 
 def check_half(t, name):
@@ -88,7 +107,9 @@ class WhisperExt:
         self.lib = _lib.lib()
 
     def _call(self, name, *args):
-        _lib.check(getattr(self.lib, name)(*args), name)
+        status = getattr(self.lib, name)(*args)
+        if status:
+            _lib.check(status, name)
 
     # ---- reference ops -------------------------------------------------------------------
     def lm_head_argmax(self, h, w, suppress, best):
@@ -112,29 +133,19 @@ class WhisperExt:
                    int(max_pos), _stream())
 
     def _attn_checks(self, q, k, v, out, len_state, k_new, v_new, part_m, part_l, part_acc, split_keys):
-        for t, n in ((q, 'q'), (k, 'k'), (v, 'v'), (out, 'out')):
-            check_half(t, n)
-        _require(k.dim() == 3 and k.size(2) == HEAD_DIM and k.shape == v.shape, 'k, v must be [heads, max_len, 64]')
-        heads, max_len = k.size(0), k.size(1)
-        splits = -(-max_len // split_keys)
-        _require(q.numel() == heads * HEAD_DIM and out.numel() == heads * HEAD_DIM, 'q, out must be [heads * 64]')
-        _require((k_new is None) == (v_new is None) == (len_state is None),
-                 'len_state, k_new and v_new must be given together')
-        if k_new is not None:
-            check_half(k_new, 'k_new')
-            check_half(v_new, 'v_new')
-            _require(k_new.numel() == heads * HEAD_DIM and v_new.numel() == heads * HEAD_DIM,
-                     'k_new, v_new must be [heads, 64]')
-            _require(len_state.dtype == torch.int64 and len_state.is_cuda, 'len_state must be CUDA int64')
-        for t in (part_m, part_l, part_acc):
-            _require(t.is_cuda and t.is_contiguous() and t.dtype == torch.float32,
-                     'workspace must be contiguous CUDA fp32')
+        heads, max_len = self._attn_io_checks(q, k, v, out, len_state, k_new, v_new)
+        if not _all_contiguous(_F32, part_m, part_l, part_acc):
+            for t in (part_m, part_l, part_acc):
+                _require(t.is_cuda and t.is_contiguous() and t.dtype == torch.float32,
+                         'workspace must be contiguous CUDA fp32')
         slots = min(part_m.numel(), part_l.numel(), part_acc.numel() // HEAD_DIM)
-        _require(slots >= heads * splits, f'workspace too small for {splits} splits')
+        splits = -(-max_len // split_keys)
+        if slots < heads * splits:
+            raise RuntimeError(f'workspace too small for {splits} splits')
         return heads, max_len, slots
 
     def decode_attention(self, q, k, v, out, len_state, k_new, v_new, part_m, part_l, part_acc, scale):
-        """whisper_kernels.cu:300-339: split kernel (64 keys per split) + combine kernel."""
+        """whisper_kernels.cu:300-339: 64 keys per split, then their combine."""
         heads, max_len, slots = self._attn_checks(q, k, v, out, len_state, k_new, v_new, part_m, part_l, part_acc,
                                                   SPLIT_KEYS)
         self._call('fw_decode_attention', q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(len_state),
@@ -143,8 +154,9 @@ class WhisperExt:
 
     def add_layernorm(self, h, x, gamma, beta, y, eps):
         """whisper_kernels.cu:341-356."""
-        for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
-            check_half(t, n)
+        if not _halves(h, gamma, beta, y):
+            for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
+                check_half(t, n)
         _require(h.numel() == HIDDEN, f'hidden size must be {HIDDEN}')
         if x is not None:
             check_half(x, 'x')
@@ -179,8 +191,9 @@ class WhisperExt:
     def ln_gemv(self, h, x, h_out, gamma, beta, eps, w, bias, out, act=ACT_NONE, embed=None, nv=1):
         """r = fp16(h + x) -> h_out; y = LN(r); out = act(w y + b). embed = (cur, state, table, pos_table).
         With nv > 1, h, x, h_out and out hold nv rows and cur nv tokens (positions state[0] + v)."""
-        for t, n in ((gamma, 'gamma'), (beta, 'beta'), (w, 'w'), (out, 'out')):
-            check_half(t, n)
+        if not _halves(gamma, beta, w, out):
+            for t, n in ((gamma, 'gamma'), (beta, 'beta'), (w, 'w'), (out, 'out')):
+                check_half(t, n)
         _require(1 <= nv <= MAX_BATCH, f'nv must be in [1, {MAX_BATCH}]')
         _require(w.dim() == 2 and w.size(1) == HIDDEN and out.numel() == nv * w.size(0), 'ln_gemv shape mismatch')
         cur = state = table = pos_table = None
@@ -209,19 +222,27 @@ class WhisperExt:
             self._call('fw_ln_gemv_batch', *args, nv, _stream())
 
     def _attn_io_checks(self, q, k, v, out, len_state, k_new, v_new):
-        for t, n in ((q, 'q'), (k, 'k'), (v, 'v'), (out, 'out')):
-            check_half(t, n)
-        _require(k.dim() == 3 and k.size(2) == HEAD_DIM and k.shape == v.shape, 'k, v must be [heads, max_len, 64]')
-        heads, max_len = k.size(0), k.size(1)
-        _require(q.numel() == heads * HEAD_DIM and out.numel() == heads * HEAD_DIM, 'q, out must be [heads * 64]')
-        _require((k_new is None) == (v_new is None) == (len_state is None),
-                 'len_state, k_new and v_new must be given together')
+        if not _halves(q, k, v, out):
+            if not _halves(q, k, v, out):
+                for t, n in ((q, 'q'), (k, 'k'), (v, 'v'), (out, 'out')):
+                    check_half(t, n)
+        shape = k.shape
+        if len(shape) != 3 or shape[2] != HEAD_DIM or v.shape != shape:
+            raise RuntimeError('k, v must be [heads, max_len, 64]')
+        heads, max_len, _ = shape
+        n = heads * HEAD_DIM
+        if q.numel() != n or out.numel() != n:
+            raise RuntimeError('q, out must be [heads * 64]')
+        if not ((k_new is None) == (v_new is None) == (len_state is None)):
+            raise RuntimeError('len_state, k_new and v_new must be given together')
         if k_new is not None:
-            check_half(k_new, 'k_new')
-            check_half(v_new, 'v_new')
-            _require(k_new.numel() == heads * HEAD_DIM and v_new.numel() == heads * HEAD_DIM,
-                     'k_new, v_new must be [heads, 64]')
-            _require(len_state.dtype == torch.int64 and len_state.is_cuda, 'len_state must be CUDA int64')
+            if not _halves(k_new, v_new):
+                check_half(k_new, 'k_new')
+                check_half(v_new, 'v_new')
+            if k_new.numel() != n or v_new.numel() != n:
+                raise RuntimeError('k_new, v_new must be [heads, 64]')
+            if len_state.dtype != _I64 or not len_state.is_cuda:
+                raise RuntimeError('len_state must be CUDA int64')
         return heads, max_len
 
     def decode_attention_fused(self, q, k, v, out, len_state, k_new, v_new, scale):
@@ -373,8 +394,9 @@ class WhisperExt:
         cur[0] at state[0] to the residual h_out and the last fc2 output x_out, K/V rows written at
         state[0]. Nothing else may run on the device meanwhile. A wait past spin_limit ticks (100 MHz)
         sets the workspace's error word; read it with decoder_step_error."""
-        for t, n in ((embed, 'embed'), (pos_embed, 'pos_embed'), (h_out, 'h_out'), (x_out, 'x_out')):
-            check_half(t, n)
+        if not _halves(embed, pos_embed, h_out, x_out):
+            for t, n in ((embed, 'embed'), (pos_embed, 'pos_embed'), (h_out, 'h_out'), (x_out, 'x_out')):
+                check_half(t, n)
         _require(embed.dim() == 2 and embed.size(1) == HIDDEN and pos_embed.dim() == 2 and pos_embed.size(1) == HIDDEN
                  and pos_embed.size(0) >= max_pos, 'embed / pos_embed must be [rows, 1280]')
         _require(h_out.numel() == HIDDEN and x_out.numel() == HIDDEN, 'h_out, x_out must be [1280]')
@@ -388,8 +410,9 @@ class WhisperExt:
 
     def final_layernorm(self, h, x, gamma, beta, y, eps):
         """The LM-head kernels' final LayerNorm (their reduction order): y = LN(fp16(h + x))."""
-        for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
-            check_half(t, n)
+        if not _halves(h, gamma, beta, y):
+            for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
+                check_half(t, n)
         if x is not None:
             check_half(x, 'x')
         _require(h.numel() == HIDDEN and y.numel() == HIDDEN, f'hidden size must be {HIDDEN}')
@@ -403,8 +426,9 @@ class WhisperExt:
     def decoder_head(self, gamma, beta, eps, w, wq, meta, suppress, tokens, y_out=None, host_tokens=None, eos=()):
         """The fw_dec_head of decoder_step (raw pointers: the tensors and host_tokens must outlive it).
         eos: up to 4 end-of-text ids at which a launch stops (set_eos changes them later)."""
-        for t, n in ((gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
-            check_half(t, n)
+        if not _halves(gamma, beta, w):
+            for t, n in ((gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
+                check_half(t, n)
         _require(w.dim() == 2 and w.size(1) == HIDDEN, f'hidden size must be {HIDDEN}')
         _check(wq, 'wq', torch.int8, 'int8')
         _check(meta, 'meta', torch.float32, 'fp32')
@@ -479,8 +503,9 @@ class WhisperExt:
     def lm_head_argmax_fused(self, h, x, gamma, beta, eps, w, suppress, best, tokens, state, cur, max_pos):
         """Final residual + LN + lm_head_argmax + argmax_finalize (finalize skipped when tokens, state and
         cur are all None)."""
-        for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
-            check_half(t, n)
+        if not _halves(h, gamma, beta, w):
+            for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
+                check_half(t, n)
         if x is not None:
             check_half(x, 'x')
         _require(w.dim() == 2 and w.size(1) == HIDDEN, f'hidden size must be {HIDDEN}')
@@ -516,8 +541,9 @@ class WhisperExt:
 
     def lm_head_argmax_q8(self, h, x, gamma, beta, eps, w, wq, meta, suppress, best, tokens, state, cur, max_pos):
         """lm_head_argmax_fused with the same result, bit for bit, from the int8 table (wq, meta) of w."""
-        for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
-            check_half(t, n)
+        if not _halves(h, gamma, beta, w):
+            for t, n in ((h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (w, 'w')):
+                check_half(t, n)
         if x is not None:
             check_half(x, 'x')
         _require(w.dim() == 2 and w.size(1) == HIDDEN, f'hidden size must be {HIDDEN}')
@@ -541,16 +567,18 @@ class WhisperExt:
         return torch.empty(int(self.lib.fw_log_mel_ws_floats(int(n_samples))), dtype=torch.float32, device=device)
 
     def _log_mel_checks(self, wave, filters, out, out16, ws):
-        _check(wave, 'wave', torch.float32, 'fp32')
-        _check(filters, 'filters', torch.float32, 'fp32')
-        _check(out, 'out', torch.float32, 'fp32')
-        _check(ws, 'ws', torch.float32, 'fp32')
+        if not _all_contiguous(_F32, wave, filters, out, ws):
+            for t, n in ((wave, 'wave'), (filters, 'filters'), (out, 'out'), (ws, 'ws')):
+                _check(t, n, torch.float32, 'fp32')
         n_frames = wave.numel() // 160
-        _require(filters.shape == (201, 128), 'filters must be [201, 128]')
-        _require(out.numel() == 128 * n_frames, f'out must be [128, {n_frames}]')
+        if filters.shape != (201, 128):
+            raise RuntimeError('filters must be [201, 128]')
+        if out.numel() != 128 * n_frames:
+            raise RuntimeError(f'out must be [128, {n_frames}]')
         if out16 is not None:
             check_half(out16, 'out16')
-            _require(out16.numel() == 128 * n_frames, f'out16 must be [{n_frames}, 128]')
+            if out16.numel() != 128 * n_frames:
+                raise RuntimeError(f'out16 must be [{n_frames}, 128]')
 
     def log_mel(self, wave, filters, out, out16, ws):
         """Log-mel of one clip: log_mel_prepare then log_mel_run."""
@@ -618,8 +646,9 @@ class WhisperExt:
                    _ptr(res), epilogue, _stream())
 
     def layernorm_rows(self, x, gamma, beta, y, eps):
-        for t, n in ((x, 'x'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
-            check_half(t, n)
+        if not _halves(x, gamma, beta, y):
+            for t, n in ((x, 'x'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
+                check_half(t, n)
         _require(x.dim() == 2 and x.size(1) == HIDDEN and y.shape == x.shape, 'layernorm_rows shape mismatch')
         self._call('fw_layernorm_rows', x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), y.data_ptr(), x.size(0),
                    HIDDEN, float(eps), _stream())
@@ -638,8 +667,9 @@ class WhisperExt:
 
     def layernorm_rows_residual(self, part, bias, h, gamma, beta, y, eps, epilogue):
         """h <- residual epilogue(part[0] + part[1], bias) in place, then y <- LN(h) (part from gemm_splitk)."""
-        for t, n in ((bias, 'bias'), (h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
-            check_half(t, n)
+        if not _halves(bias, h, gamma, beta, y):
+            for t, n in ((bias, 'bias'), (h, 'h'), (gamma, 'gamma'), (beta, 'beta'), (y, 'y')):
+                check_half(t, n)
         _check(part, 'part', torch.float32, 'float32')
         rows = h.size(0)
         _require(h.dim() == 2 and h.size(1) == HIDDEN and y.shape == h.shape and part.shape == (2, rows, HIDDEN),
@@ -659,8 +689,9 @@ class WhisperExt:
 
     def encoder_qkv(self, y, w, bias, qkv, vt, heads):
         """q/k/v projection of an encoder layer: q (scaled by 1/8) and k into qkv, v into vt."""
-        for t, n in ((y, 'y'), (w, 'w'), (qkv, 'qkv')):
-            check_half(t, n)
+        if not _halves(y, w, qkv):
+            for t, n in ((y, 'y'), (w, 'w'), (qkv, 'qkv')):
+                check_half(t, n)
         seq, d = y.shape
         _require(d == heads * HEAD_DIM and w.shape == (3 * d, d) and qkv.shape == (seq, 3 * d),
                  'encoder_qkv shape mismatch')

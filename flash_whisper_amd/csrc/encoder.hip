@@ -3,6 +3,8 @@
 // self-attention is in attention_enc.hip. Semantics follow HF WhisperEncoder.forward in fp16
 // (transformers models/whisper/modeling_whisper.py:592-648, layer :379-414, attention :284-358):
 // every op output is rounded to fp16, accumulation is fp32.
+#include <type_traits>
+
 #include "lds_pipe.h"
 
 namespace fw {
@@ -120,41 +122,32 @@ __device__ __forceinline__ float gelu_enc(float x) {
   return x * (x >= 0.0f ? 1.0f - c : c);
 }
 
-// Output value before the final fp16 rounding; `res` is the residual / position operand of the
-// epilogues that read one.
-__device__ __forceinline__ float epilogue_apply(int epi, float acc, float b, float res, int col, int q_cols) {
+// The epilogue's value before its residual / position operand: an fp16 number for the epilogues that read
+// one, so it can be staged as fp16 without a rounding of its own.
+template <int EPI>
+__device__ __forceinline__ float epilogue_pre(float acc, float b, int col, int q_cols) {
   float v = round_h(acc + b);
-  switch (epi) {
-    case FW_EPI_BIAS_GELU:
-      v = gelu_enc(v);
-      break;
-    case FW_EPI_BIAS_RESID:
-      v = res + v;
-      break;
-    case FW_EPI_BIAS_RESID_CLAMP: {
-      v = round_h(res + v);
-      const float c = 65504.0f - 1000.0f;
-      v = fminf(fmaxf(v, -c), c);
-      break;
-    }
-    case FW_EPI_BIAS_GELU_POS:
-      v = round_h(gelu_enc(v)) + res;
-      break;
-    case FW_EPI_SCALE_Q:
-    case kEpiQkvVt:
-      if (col < q_cols) v = v * 0.125f;
-      break;
-    default:
-      break;
+  if constexpr (EPI == FW_EPI_BIAS_GELU) v = gelu_enc(v);
+  if constexpr (EPI == FW_EPI_BIAS_GELU_POS) v = round_h(gelu_enc(v));
+  if constexpr (EPI == FW_EPI_SCALE_Q || EPI == kEpiQkvVt)
+    if (col < q_cols) v = v * 0.125f;
+  return v;
+}
+// The value before the final fp16 rounding, from epilogue_pre's and the operand.
+template <int EPI>
+__device__ __forceinline__ float epilogue_res(float v, float res) {
+  v = res + v;
+  if constexpr (EPI == FW_EPI_BIAS_RESID_CLAMP) {
+    const float c = 65504.0f - 1000.0f;
+    v = fminf(fmaxf(round_h(v), -c), c);
   }
   return v;
 }
 
-__device__ __forceinline__ float epilogue_value(int epi, float acc, float b, const GemmArgs& g, int row, int col) {
-  const float res = epi_reads_res(epi) ? h2f(g.res[static_cast<size_t>(row) * g.ldr + col]) : 0.f;
-  return epilogue_apply(epi, acc, b, res, col, g.q_cols);
-}
-
+// Rows of fp16 outputs and operands are moved 16 bytes at a time whatever their alignment (the hardware
+// takes unaligned global accesses; the encoder's own are aligned).
+typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
+typedef _Float16 h4u __attribute__((ext_vector_type(4), aligned(2)));
 
 // MFMA operand fragments of one 64-wide k stage for a wave: A rows wm + 32 i + lane % 32, B rows
 // wn + 32 j + lane % 32, k-step s covering k 16 s .. 16 s + 15.
@@ -197,7 +190,7 @@ __device__ __forceinline__ void load_frags(const char* stage, const FragOffsets&
 
 // kT: accumulate the transposed tile (W rows as the MFMA A operand), so that acc[i][j][r] holds
 // C[32 i + lane % 32][32 j + 8 (r / 4) + 4 g + r % 4]: four adjacent output columns per lane, which
-// the epilogue then reads and writes as one 8-byte access.
+// the epilogue stages as one 8-byte (fp32 sums: 16-byte) LDS access.
 template <int kTM, int kTN, bool kT>
 __device__ __forceinline__ void mma_frags(const Frags<kTM, kTN>& f, f16v (&acc)[kTM][kTN]) {
 #pragma unroll
@@ -349,11 +342,11 @@ __device__ __forceinline__ void dma_stage_s(const GemmArgs& g, const CopyOffsets
 // into a [128 columns][BM] staging tile, already in vt_pos order (tiles start at multiples of 64 and
 // vt_pos permutes within 16-key groups), and the block then writes each column's BM keys as whole
 // 16-byte chunks instead of one 8-byte store per 4 keys and column.
-template <int BM, int kTM, int kTN>
+template <int BM, int kTM, int kTN, int ST>
 __device__ __forceinline__ void store_vt(const GemmArgs& g, const f16v (&acc)[kTM][kTN], int m0, int n0, int wm,
                                          int wn, int lr, int lg, u32x4* lds) {
   constexpr int kStride = BM + 8;  // halves per staged column (16-byte aligned rows)
-  static_assert(kBN * kStride * 2 <= dma_stages<BM>() * (BM + kBN) * 128, "staging tile must fit the ring");
+  static_assert(kBN * kStride * 2 <= ST * (BM + kBN) * 128, "staging tile must fit the ring");
   _Float16* t = reinterpret_cast<_Float16*>(lds);
   __syncthreads();  // every wave has read its last operand fragments from the ring
 #pragma unroll
@@ -390,9 +383,6 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArg
   static_assert(kWM % 32 == 0 && kTN >= 1 && BM % (8 * kNW) == 0, "wave tiling");
   constexpr int kStageBytes = (BM + kBN) * 128;
   constexpr int kPerStage = (BM / 8 / kNW) + (kBN / 8 / kNW);  // copies per thread per stage
-  // Transposed accumulators (8-byte epilogue accesses) pay off on the 64-row tiles of the 1280-column
-  // GEMMs (fc2 44 -> 39 us, out projection 16 -> 13 us); on 256-row tiles they measured slower.
-  constexpr bool kT = BM == 64 && EPI != kEpiQkvVt;
   __shared__ __align__(1024) u32x4 lds[kDmaStages * kStageBytes / 16];
 
   int m0, n0;
@@ -432,91 +422,107 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArg
 #pragma unroll
   for (int s = 0; s < kDmaStages; ++s)
     if (s < kt_n) issue(s, s);
-  Frags<kTM, kTN> fa, fb;
-  // this thread's copies of stage kt have landed once at most the later issued stages remain
-  wait_stages_ahead<kPerStage, kDmaStages - 1>(min(kDmaStages - 1, kt_n - 1));
-  barrier_only();
-  load_frags<kTM, kTN>(lds_bytes, fo, fa);
-  int cur = 0;  // ring slot of stage kt
-  // stage kt with a stage kt + 1 after it
-  auto step = [&](int kt, const Frags<kTM, kTN>& frags_kt, Frags<kTM, kTN>& nxt) {
-    wait_stages_ahead<kPerStage, kDmaStages - 1>(min(kDmaStages - 2, kt_n - 2 - kt));
-    lds_barrier();  // own fragment reads of stage kt done; stage kt + 1 visible; slot kt free
-    if (kt + kDmaStages < kt_n) issue(kt + kDmaStages, cur);
-    cur = cur + 1 == kDmaStages ? 0 : cur + 1;
-    load_frags<kTM, kTN>(lds_bytes + cur * kStageBytes, fo, nxt);
-    mma_frags<kTM, kTN, kT>(frags_kt, acc);
+  auto main_loop = [&](auto transposed) {
+    constexpr bool kT = decltype(transposed)::value;
+    Frags<kTM, kTN> fa, fb;
+    // this thread's copies of stage kt have landed once at most the later issued stages remain
+    wait_stages_ahead<kPerStage, kDmaStages - 1>(min(kDmaStages - 1, kt_n - 1));
+    barrier_only();
+    load_frags<kTM, kTN>(lds_bytes, fo, fa);
+    int cur = 0;  // ring slot of stage kt
+    // stage kt with a stage kt + 1 after it
+    auto step = [&](int kt, const Frags<kTM, kTN>& frags_kt, Frags<kTM, kTN>& nxt) {
+      wait_stages_ahead<kPerStage, kDmaStages - 1>(min(kDmaStages - 2, kt_n - 2 - kt));
+      lds_barrier();  // own fragment reads of stage kt done; stage kt + 1 visible; slot kt free
+      if (kt + kDmaStages < kt_n) issue(kt + kDmaStages, cur);
+      cur = cur + 1 == kDmaStages ? 0 : cur + 1;
+      load_frags<kTM, kTN>(lds_bytes + cur * kStageBytes, fo, nxt);
+      mma_frags<kTM, kTN, kT>(frags_kt, acc);
+    };
+    int kt = 0;
+    for (; kt + 2 < kt_n; kt += 2) {
+      step(kt, fa, fb);
+      step(kt + 1, fb, fa);
+    }
+    if (kt + 1 < kt_n) {
+      step(kt, fa, fb);
+      mma_frags<kTM, kTN, kT>(fb, acc);
+    } else {
+      mma_frags<kTM, kTN, kT>(fa, acc);
+    }
   };
-  int kt = 0;
-  for (; kt + 2 < kt_n; kt += 2) {
-    step(kt, fa, fb);
-    step(kt + 1, fb, fa);
+  if constexpr (EPI == kEpiQkvVt) {
+    if (n0 >= 2 * g.q_cols) {  // a v column tile (q_cols % 128 == 0): the branch is uniform per block
+      main_loop(std::false_type{});
+      store_vt<BM, kTM, kTN, kDmaStages>(g, acc, m0, n0, wm, wn, lr, lg, lds);
+      return;
+    }
   }
-  if (kt + 1 < kt_n) {
-    step(kt, fa, fb);
-    mma_frags<kTM, kTN, kT>(fb, acc);
-  } else {
-    mma_frags<kTM, kTN, kT>(fa, acc);
-  }
+  main_loop(std::true_type{});
+  __syncthreads();  // every wave has read its last operand fragments from the ring
 
-  if constexpr (kT) {
+  // The tile goes through LDS, so that its rows are written (and the residual's read) 256 bytes at a time:
+  // the accumulators give a lane 4 adjacent columns of a row at best, whose stores spread over 32 rows.
+  // Against storing from the registers (2 bytes of a column each, 8 bytes on 64-row tiles): a product with
+  // a single k stage 4.3 -> 3.8 us at 1500 x 1280, 6.1 -> 5.8 us at 1500 x 3840, 7.45 us as before at
+  // 1500 x 5120, where writing 15 MB takes that long either way; the encoder 4034 -> 4012 us.
+  if constexpr (EPI == kEpiPartial) {
+    constexpr int kRowF = kBN + 4;
+    static_assert(BM * kRowF * 4 <= kDmaStages * kStageBytes, "staging tile must fit the ring");
+    float* t = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int i = 0; i < kTM; ++i)
+#pragma unroll
+      for (int j = 0; j < kTN; ++j)
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+          f4v v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * rq + e];
+          *reinterpret_cast<f4v*>(t + (wm + 32 * i + lr) * kRowF + wn + 32 * j + 8 * rq + 4 * lg) = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int c = tid; c < BM * (kBN / 4); c += kNW * 64) {
+      const int row = c / (kBN / 4), col = c % (kBN / 4) * 4;
+      if (m0 + row < g.m)
+        *reinterpret_cast<f4v*>(g.part + (static_cast<size_t>(split) * g.m + m0 + row) * g.n + n0 + col) =
+            *reinterpret_cast<const f4v*>(t + row * kRowF + col);
+    }
+  } else {
+    constexpr int kRowH = kBN + 8;  // 16-byte aligned rows
+    static_assert(BM * kRowH * 2 <= kDmaStages * kStageBytes, "staging tile must fit the ring");
+    _Float16* t = reinterpret_cast<_Float16*>(lds);
 #pragma unroll
     for (int j = 0; j < kTN; ++j)
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq) {
-        const int col = n0 + wn + 32 * j + 8 * rq + 4 * lg;  // columns col .. col + 3
-        h4v bb = {};
-        if (g.bias) bb = *reinterpret_cast<const h4v*>(g.bias + col);
+        const int cl = wn + 32 * j + 8 * rq + 4 * lg;  // columns cl .. cl + 3 of the tile
+        h4u bb = {};
+        if (g.bias) bb = *reinterpret_cast<const h4u*>(g.bias + n0 + cl);
 #pragma unroll
         for (int i = 0; i < kTM; ++i) {
-          const int row = m0 + wm + 32 * i + lr;
-          if (row < g.m) {
-            h4v o;
-            if constexpr (EPI == kEpiCrossKV) {
+          h4v o;
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o[e] = f2h(acc[i][j][4 * rq + e] + h2f(bb[e]));
-              const int d = col & 63, lhk = col >> 6;
-              *reinterpret_cast<h4v*>(g.out + (static_cast<size_t>(lhk) * g.t_len + row) * 64 + d) = o;
-            } else {
-              h4v rv = {};
-              if constexpr (epi_reads_res(EPI)) rv = *reinterpret_cast<const h4v*>(g.res + static_cast<size_t>(row) * g.ldr + col);
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                o[e] = f2h(epilogue_apply(EPI, acc[i][j][4 * rq + e], h2f(bb[e]), h2f(rv[e]), col + e, g.q_cols));
-              *reinterpret_cast<h4v*>(g.out + static_cast<size_t>(row) * g.ldo + col) = o;
-            }
-          }
+          for (int e = 0; e < 4; ++e)
+            o[e] = f2h(epilogue_pre<EPI>(acc[i][j][4 * rq + e], h2f(bb[e]), n0 + cl + e, g.q_cols));
+          *reinterpret_cast<h4v*>(t + (wm + 32 * i + lr) * kRowH + cl) = o;
         }
       }
-    return;
-  }
-  if constexpr (EPI == kEpiQkvVt) {
-    if (n0 >= 2 * g.q_cols) {  // a v column tile (q_cols % 128 == 0): the branch is uniform per block
-      store_vt<BM, kTM, kTN>(g, acc, m0, n0, wm, wn, lr, lg, lds);
-      return;
-    }
-  }
+    __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kTN; ++j) {
-    const int col = n0 + wn + 32 * j + lr;
-    const float b = g.bias ? h2f(g.bias[col]) : 0.f;
+    for (int c = tid; c < BM * (kBN / 8); c += kNW * 64) {
+      const int rl = c / (kBN / 8), cl = c % (kBN / 8) * 8, row = m0 + rl, col = n0 + cl;
+      if (row >= g.m) continue;
+      h8v v = *reinterpret_cast<const h8v*>(t + rl * kRowH + cl);
+      if constexpr (epi_reads_res(EPI)) {
+        const h8u r = *reinterpret_cast<const h8u*>(g.res + static_cast<size_t>(row) * g.ldr + col);
 #pragma unroll
-    for (int i = 0; i < kTM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lg + (r & 3);
-        if (row < g.m) {
-          if constexpr (EPI == kEpiPartial) {
-            g.part[(static_cast<size_t>(split) * g.m + row) * g.n + col] = acc[i][j][r];
-          } else if constexpr (EPI == kEpiCrossKV) {
-            const int d = col & 63, lhk = col >> 6;
-            const size_t o = (static_cast<size_t>(lhk) * g.t_len + row) * 64 + d;
-            g.out[o] = f2h(acc[i][j][r] + b);
-          } else {
-            g.out[static_cast<size_t>(row) * g.ldo + col] = f2h(epilogue_value(EPI, acc[i][j][r], b, g, row, col));
-          }
-        }
+        for (int e = 0; e < 8; ++e) v[e] = f2h(epilogue_res<EPI>(h2f(v[e]), h2f(r[e])));
       }
+      _Float16* dst = EPI == kEpiCrossKV ? g.out + (static_cast<size_t>(col >> 6) * g.t_len + row) * 64 + (col & 63)
+                                         : g.out + static_cast<size_t>(row) * g.ldo + col;
+      *reinterpret_cast<h8u*>(dst) = v;
     }
   }
 }
@@ -686,16 +692,22 @@ __global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(GemmArgs g) {
     if constexpr (EPI == kEpiPartial) {
       *reinterpret_cast<f4v*>(g.part + (static_cast<size_t>(split) * g.m + row) * g.n + col) = v;
     } else {
-      h4v bb = {}, rv = {}, o;
-      if (g.bias) bb = *reinterpret_cast<const h4v*>(g.bias + col);
-      if constexpr (epi_reads_res(EPI)) rv = *reinterpret_cast<const h4v*>(g.res + static_cast<size_t>(row) * g.ldr + col);
+      h4u bb = {};
+      h4v o;
+      if (g.bias) bb = *reinterpret_cast<const h4u*>(g.bias + col);
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o[e] = f2h(epilogue_apply(EPI, v[e], h2f(bb[e]), h2f(rv[e]), col + e, g.q_cols));
+      for (int e = 0; e < 4; ++e) v[e] = epilogue_pre<EPI>(v[e], h2f(bb[e]), col + e, g.q_cols);
+      if constexpr (epi_reads_res(EPI)) {
+        const h4u rv = *reinterpret_cast<const h4u*>(g.res + static_cast<size_t>(row) * g.ldr + col);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = epilogue_res<EPI>(v[e], h2f(rv[e]));
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = f2h(v[e]);
       if constexpr (EPI == kEpiCrossKV)
-        *reinterpret_cast<h4v*>(g.out + (static_cast<size_t>(col >> 6) * g.t_len + row) * 64 + (col & 63)) = o;
+        *reinterpret_cast<h4u*>(g.out + (static_cast<size_t>(col >> 6) * g.t_len + row) * 64 + (col & 63)) = o;
       else
-        *reinterpret_cast<h4v*>(g.out + static_cast<size_t>(row) * g.ldo + col) = o;
+        *reinterpret_cast<h4u*>(g.out + static_cast<size_t>(row) * g.ldo + col) = o;
     }
   }
 }
@@ -823,17 +835,9 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
   return best;
 }
 
-// The sliced kernel's and the 64-row tiles' epilogues move 4 adjacent columns at a time.
-bool vector_epilogue(const GemmArgs& g) {
-  const uintptr_t p = reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.out) | reinterpret_cast<uintptr_t>(g.res);
-  return !(p & 7u);
-}
-
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
-  const bool vec = vector_epilogue(g), qkv = epi == kEpiQkvVt;
-  // (the 64-row tiles store q/k/v by element, so they need no alignment there)
-  switch (choose_tile(g, [&](Tile t) { return vec || t < kD64 || (qkv && t == kD64); })) {
+  switch (choose_tile(g, [](Tile) { return true; })) {
     case kD256: return launch_dma<256, false>(g, epi, s);
     case kD192: return launch_dma<192, false>(g, epi, s);
     case kD64: return launch_dma<64, false>(g, epi, s);
@@ -850,12 +854,12 @@ int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
 // CU, so that one's epilogue runs beside the other's copies (3000 rows: 9.9 us against 12.6 for a
 // register-staged gather, 10.3 for a 2-deep ring and 10.1 for 128-row tiles; 1000 rows: 6.7, 10.5, 7.8, 9.4).
 int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
-  const bool vec = vector_epilogue(g) && copy_offsets_fit(g);  // (the sliced kernel's weight offsets are 32-bit)
-  const Tile t = choose_tile(g, [&](Tile c) { return c == kD128 || (vec && c >= kD64); });
+  const bool fit = copy_offsets_fit(g);  // the sliced kernel's weight offsets are 32-bit
+  const Tile t = choose_tile(g, [&](Tile c) { return c == kD128 || c == kD64 || (fit && c > kD64); });
   if (t == kS64x64) return launch_ks<64, 64, true>(g, epi, s);
   if (t == kS64x32) return launch_ks<64, 32, true>(g, epi, s);
   if (t == kS32x32) return launch_ks<32, 32, true>(g, epi, s);
-  if (vec && g.k < 1024) return launch_dma<64, true, 3>(g, epi, s);
+  if (g.k < 1024) return launch_dma<64, true, 3>(g, epi, s);
   if (t == kS96x64) return launch_ks<96, 64, true>(g, epi, s);
   if (t == kD64) return launch_dma<64, true>(g, epi, s);
   return launch_dma<128, true>(g, epi, s);

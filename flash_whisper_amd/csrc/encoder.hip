@@ -260,29 +260,25 @@ constexpr int gemm_wave_cols() { return BM == 192 || (BM == 64 && FW_W64 == 8) ?
 // Source of the implicit conv's zero padding rows: a k stage of one A row is 64 halves.
 __device__ __align__(16) _Float16 g_zero_row[kBK];
 
-// CONV: implicit conv1d (k = 3, pad 1). A 64-wide k stage lies inside one tap (c_in % 64 == 0), so A
-// row m of the stage is 64 contiguous channels of input row m * stride + tap - 1, or zeros outside
+// Implicit conv1d (k = 3, pad 1) of any size: a 64-wide k stage lies inside one tap (c_in % 64 == 0), so
+// A row m of the stage is 64 contiguous channels of input row m * stride + tap - 1, or zeros outside
 // [0, t_in).
-template <int BM, bool CONV = false>
-__device__ __forceinline__ void dma_stage(const GemmArgs& g, int m0, int n0, int k0, int wave, int lane,
+template <int BM>
+__device__ __forceinline__ void dma_stage_conv(const GemmArgs& g, int m0, int n0, int k0, int wave, int lane,
                                           uint32_t lds_stage) {
   constexpr int kAInstr = BM / 8 / gemm_waves<BM>();  // wave instructions per A tile (8 rows each), per wave
   constexpr int kBInstr = kBN / 8 / gemm_waves<BM>();
   const int rsub = lane >> 3, slot = lane & 7;
-  const int tap = CONV ? k0 / g.c_in : 0, ch0 = CONV ? k0 - tap * g.c_in : 0;
+  const int tap = k0 / g.c_in, ch0 = k0 - tap * g.c_in;
 #pragma unroll
   for (int i = 0; i < kAInstr; ++i) {
     const int blk = wave * kAInstr + i;  // 8-row block of the tile
     const int row = blk * 8 + rsub;
     const int gm = min(m0 + row, g.m - 1);  // rows past m are computed and never stored
     const int chunk = swz_slot(row, slot);
-    const _Float16* src;
-    if constexpr (CONV) {
-      const int r = gm * g.conv_stride + tap - 1;
-      src = (r >= 0 && r < g.t_in) ? g.a + static_cast<size_t>(r) * g.c_in + ch0 + chunk * 8 : g_zero_row + chunk * 8;
-    } else {
-      src = g.a + static_cast<size_t>(gm) * g.lda + k0 + chunk * 8;
-    }
+    const int r = gm * g.conv_stride + tap - 1;
+    const _Float16* src =
+        (r >= 0 && r < g.t_in) ? g.a + static_cast<size_t>(r) * g.c_in + ch0 + chunk * 8 : g_zero_row + chunk * 8;
     dma16(src, __builtin_amdgcn_readfirstlane(lds_stage + blk * 1024));
   }
 #pragma unroll
@@ -324,16 +320,48 @@ __device__ __forceinline__ void copy_offsets(const GemmArgs& g, int m0, int n0, 
   }
 }
 
+// Implicit convs: row m, tap, channel ch of A is input row m * stride + tap - 1, that is x[m * stride *
+// c_in - c_in + kk] at column kk = tap * c_in + ch. So A is a matrix of pitch stride * c_in that starts one
+// input row early, and a copy's source is again a per-lane offset plus a scalar one. Only row 0 at the
+// first tap and the last input row's successor at the third fall outside x: their lanes' offsets point past
+// the buffer's end there, which reads as zero (3000 -> 1500 x 1280, k = 3840: 29.5 against 31.6 us with the
+// source row worked out, compared and selected for every copy). Buffers of less than 2 GiB only.
+struct ConvSource {
+  buffer_rsrc x;
+  __device__ __forceinline__ explicit ConvSource(const GemmArgs& g)
+      : x(make_rsrc(g.a - g.c_in, static_cast<uint32_t>(g.t_in + 1) * g.c_in * 2)) {}
+  // this lane's chunk of A row gm, LDS row `row`, slot `slot`: its offset at each tap
+  __device__ __forceinline__ static void offsets(const GemmArgs& g, int gm, int row, int slot, uint32_t (&o)[3]) {
+    const int r = gm * g.conv_stride;
+    o[1] = static_cast<uint32_t>((r * g.c_in + swz_slot(row, slot) * 8) * 2);
+    o[0] = r > 0 ? o[1] : kPastEnd;
+    o[2] = r + 1 < g.t_in ? o[1] : kPastEnd;
+  }
+  __device__ __forceinline__ void copy(const uint32_t (&o)[3], int tap, uint32_t kk, uint32_t lds_base) const {
+    dma16_buf(tap == 0 ? o[0] : tap == 1 ? o[1] : o[2], x, kk * 2, lds_base);
+  }
+};
+bool conv_offsets_fit(const GemmArgs& g) {
+  return (static_cast<size_t>(g.t_in) + 1) * g.c_in * 2 < kPastEnd;
+}
+
+template <int BM, int kNW>
+__device__ __forceinline__ void dma_stage_w(const GemmArgs& g, const CopyOffsets<BM, kNW>& c, int kt, int wave,
+                                            uint32_t lds_stage) {
+  using C = CopyOffsets<BM, kNW>;
+  const char* wb = reinterpret_cast<const char*>(g.w) + static_cast<size_t>(kt) * (kBK * 2);
+#pragma unroll
+  for (int i = 0; i < C::kB; ++i) dma16_s(c.b[i], wb, lds_stage + BM * 128 + (wave * C::kB + i) * 1024);
+}
+
 template <int BM, int kNW>
 __device__ __forceinline__ void dma_stage_s(const GemmArgs& g, const CopyOffsets<BM, kNW>& c, int kt, int wave,
                                             uint32_t lds_stage) {
   using C = CopyOffsets<BM, kNW>;
   const char* ab = reinterpret_cast<const char*>(g.a) + static_cast<size_t>(kt) * (kBK * 2);
-  const char* wb = reinterpret_cast<const char*>(g.w) + static_cast<size_t>(kt) * (kBK * 2);
 #pragma unroll
   for (int i = 0; i < C::kA; ++i) dma16_s(c.a[i], ab, lds_stage + (wave * C::kA + i) * 1024);
-#pragma unroll
-  for (int i = 0; i < C::kB; ++i) dma16_s(c.b[i], wb, lds_stage + BM * 128 + (wave * C::kB + i) * 1024);
+  dma_stage_w<BM, kNW>(g, c, kt, wave, lds_stage);
 }
 
 // v columns of the q/k/v projection -> vt[head * 64 + d][vt_pos(t)]; rows in [m, vt_pad) get zeros so
@@ -376,7 +404,9 @@ __device__ __forceinline__ void store_vt(const GemmArgs& g, const f16v (&acc)[kT
   }
 }
 
-template <int BM, int EPI, bool CONV = false, int ST = dma_stages<BM>()>
+constexpr int kNoConv = 0, kConvBuffer = 1, kConvAny = 2;  // conv sources through a buffer, or worked out for any size
+
+template <int BM, int EPI, int CONV = kNoConv, int ST = dma_stages<BM>()>
 __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArgs g) {
   constexpr int kDmaStages = ST, kNW = gemm_waves<BM>(), kNWN = gemm_wave_cols<BM>();
   constexpr int kWM = BM / (kNW / kNWN), kTM = kWM / 32, kTN = kBN / kNWN / 32;
@@ -409,14 +439,30 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(GemmArg
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
   CopyOffsets<BM, kNW> co;
-  if constexpr (!CONV) copy_offsets<BM, kNW>(g, m0, n0, wave, lane, co);
+  copy_offsets<BM, kNW>(g, m0, n0, wave, lane, co);
+  const ConvSource src(g);
+  uint32_t conv_a[BM / 8 / kNW][3];
+  if constexpr (CONV == kConvBuffer) {
+#pragma unroll
+    for (int i = 0; i < BM / 8 / kNW; ++i) {
+      const int row = (wave * (BM / 8 / kNW) + i) * 8 + (lane >> 3);
+      ConvSource::offsets(g, min(m0 + row, g.m - 1), row, lane & 7, conv_a[i]);
+    }
+  }
   const FragOffsets fo = frag_offsets<BM>(wm, wn, lr, lg);
   auto issue = [&](int kt, int ring_slot) {  // stage kt's copies into ring slot ring_slot
     const uint32_t dst = lds0 + ring_slot * kStageBytes;
-    if constexpr (CONV)
-      dma_stage<BM, true>(g, m0, n0, kt * kBK, wave, lane, dst);
-    else
+    if constexpr (CONV == kConvAny) {
+      dma_stage_conv<BM>(g, m0, n0, kt * kBK, wave, lane, dst);
+    } else if constexpr (CONV == kConvBuffer) {
+      const int tap = kt * kBK / g.c_in;
+#pragma unroll
+      for (int i = 0; i < BM / 8 / kNW; ++i)
+        src.copy(conv_a[i], tap, kt * kBK, dst + (wave * (BM / 8 / kNW) + i) * 1024);
+      dma_stage_w<BM, kNW>(g, co, kt, wave, dst);
+    } else {
       dma_stage_s<BM, kNW>(g, co, kt, wave, dst);
+    }
   };
   const int kt_n = g.k / kBK;
 #pragma unroll
@@ -566,13 +612,15 @@ __global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(GemmArgs g) {
   const uint32_t ring0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
 
   // byte offsets of this lane's chunk of every copy of a stage (A rows, then W rows)
-  uint32_t aoff[TM / 8], woff[TN / 8];
-  if constexpr (!CONV) {
+  uint32_t aoff[TM / 8][3], woff[TN / 8];
+  const ConvSource src(g);
 #pragma unroll
-    for (int i = 0; i < TM / 8; ++i) {
-      const int row = i * 8 + rsub;
-      aoff[i] = static_cast<uint32_t>((static_cast<size_t>(min(m0 + row, g.m - 1)) * g.lda + swz_slot(row, slot8) * 8) * 2);
-    }
+  for (int i = 0; i < TM / 8; ++i) {
+    const int row = i * 8 + rsub, gm = min(m0 + row, g.m - 1);
+    if constexpr (CONV)
+      ConvSource::offsets(g, gm, row, slot8, aoff[i]);
+    else
+      aoff[i][0] = static_cast<uint32_t>((static_cast<size_t>(gm) * g.lda + swz_slot(row, slot8) * 8) * 2);
   }
 #pragma unroll
   for (int i = 0; i < TN / 8; ++i) {
@@ -583,17 +631,12 @@ __global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(GemmArgs g) {
     const uint32_t dst = __builtin_amdgcn_readfirstlane(ring0 + slot * kStageBytes);
     const size_t kb = static_cast<size_t>(kt) * (kBK * 2);
     if constexpr (CONV) {
-      const int tap = kt * kBK / g.c_in, ch0 = kt * kBK - tap * g.c_in;
+      const int tap = kt * kBK / g.c_in;
 #pragma unroll
-      for (int i = 0; i < TM / 8; ++i) {
-        const int row = i * 8 + rsub;
-        const int r = min(m0 + row, g.m - 1) * g.conv_stride + tap - 1;
-        const _Float16* src = (r >= 0 && r < g.t_in) ? g.a + static_cast<size_t>(r) * g.c_in + ch0 : g_zero_row;
-        dma16(src + swz_slot(row, slot8) * 8, dst + i * 1024);
-      }
+      for (int i = 0; i < TM / 8; ++i) src.copy(aoff[i], tap, kt * kBK, dst + i * 1024);
     } else {
 #pragma unroll
-      for (int i = 0; i < TM / 8; ++i) dma16_s(aoff[i], reinterpret_cast<const char*>(g.a) + kb, dst + i * 1024);
+      for (int i = 0; i < TM / 8; ++i) dma16_s(aoff[i][0], reinterpret_cast<const char*>(g.a) + kb, dst + i * 1024);
     }
 #pragma unroll
     for (int i = 0; i < TN / 8; ++i)
@@ -743,14 +786,14 @@ bool copy_offsets_fit(const GemmArgs& g) {
          (static_cast<size_t>(g.n - 1) * g.ldw + kBK) * 2 < kLimit;
 }
 
-template <int BM, bool CONV, int ST = dma_stages<BM>()>
+template <int BM, int CONV, int ST = dma_stages<BM>()>
 int launch_dma(GemmArgs g, int epi, hipStream_t s) {
   const dim3 grid((g.n / kBN) * ((g.m + BM - 1) / BM)), block(gemm_waves<BM>() * 64);
   choose_xcd_groups(g, BM);
   switch (epi) {
 #define FW_GEMM_CASE(E, C) \
   case E:                  \
-    if constexpr (C || !CONV) hipLaunchKernelGGL((gemm_dma_kernel<BM, E, CONV, ST>), grid, block, 0, s, g); \
+    if constexpr (C || CONV == kNoConv) hipLaunchKernelGGL((gemm_dma_kernel<BM, E, CONV, ST>), grid, block, 0, s, g); \
     break;
     FW_GEMM_CASE(FW_EPI_BIAS, true)
     FW_GEMM_CASE(FW_EPI_BIAS_GELU, true)
@@ -838,14 +881,14 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
   switch (choose_tile(g, [](Tile) { return true; })) {
-    case kD256: return launch_dma<256, false>(g, epi, s);
-    case kD192: return launch_dma<192, false>(g, epi, s);
-    case kD64: return launch_dma<64, false>(g, epi, s);
+    case kD256: return launch_dma<256, kNoConv>(g, epi, s);
+    case kD192: return launch_dma<192, kNoConv>(g, epi, s);
+    case kD64: return launch_dma<64, kNoConv>(g, epi, s);
     case kS96x64: return launch_ks<96, 64, false>(g, epi, s);
     case kS64x64: return launch_ks<64, 64, false>(g, epi, s);
     case kS64x32: return launch_ks<64, 32, false>(g, epi, s);
     case kS32x32: return launch_ks<32, 32, false>(g, epi, s);
-    default: return launch_dma<128, false>(g, epi, s);
+    default: return launch_dma<128, kNoConv>(g, epi, s);
   }
 }
 
@@ -854,15 +897,21 @@ int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
 // CU, so that one's epilogue runs beside the other's copies (3000 rows: 9.9 us against 12.6 for a
 // register-staged gather, 10.3 for a 2-deep ring and 10.1 for 128-row tiles; 1000 rows: 6.7, 10.5, 7.8, 9.4).
 int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
-  const bool fit = copy_offsets_fit(g);  // the sliced kernel's weight offsets are 32-bit
-  const Tile t = choose_tile(g, [&](Tile c) { return c == kD128 || c == kD64 || (fit && c > kD64); });
-  if (t == kS64x64) return launch_ks<64, 64, true>(g, epi, s);
-  if (t == kS64x32) return launch_ks<64, 32, true>(g, epi, s);
-  if (t == kS32x32) return launch_ks<32, 32, true>(g, epi, s);
-  if (g.k < 1024) return launch_dma<64, true, 3>(g, epi, s);
-  if (t == kS96x64) return launch_ks<96, 64, true>(g, epi, s);
-  if (t == kD64) return launch_dma<64, true>(g, epi, s);
-  return launch_dma<128, true>(g, epi, s);
+  if (!conv_offsets_fit(g) || !copy_offsets_fit(g)) return launch_dma<128, kConvAny>(g, epi, s);
+  switch (choose_tile(g, [&](Tile t) { return t >= kD128; })) {
+    case kS64x64: return launch_ks<64, 64, true>(g, epi, s);
+    case kS64x32: return launch_ks<64, 32, true>(g, epi, s);
+    case kS32x32: return launch_ks<32, 32, true>(g, epi, s);
+    case kS96x64:
+      if (g.k >= 1024) return launch_ks<96, 64, true>(g, epi, s);
+      break;
+    case kD64:
+      if (g.k >= 1024) return launch_dma<64, kConvBuffer>(g, epi, s);
+      break;
+    default:
+      if (g.k >= 1024) return launch_dma<128, kConvBuffer>(g, epi, s);
+  }
+  return launch_dma<64, kConvBuffer, 3>(g, epi, s);
 }
 
 // ------------------------------------------------------------------------------------------

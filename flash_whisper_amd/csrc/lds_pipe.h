@@ -37,6 +37,19 @@ __device__ __forceinline__ void dma16_s(uint32_t voff, const void* sbase, uint32
   asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_base)
                : "memory", "m0");
 }
+// The same copy through a raw buffer: a lane whose offset lies past the buffer's end fills its chunk with
+// zeros. `soff` moves all lanes and counts against the end too.
+typedef unsigned int buffer_rsrc __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ buffer_rsrc make_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t p = reinterpret_cast<uint64_t>(base);
+  // raw buffer: stride 0 (so offsets and the end are in bytes), 32-bit data format
+  return buffer_rsrc{static_cast<uint32_t>(p), static_cast<uint32_t>(p >> 32) & 0xFFFFu, bytes, 0x00020000u};
+}
+constexpr uint32_t kPastEnd = 0x80000000u;  // an offset past the end of any buffer of less than 2 GiB
+__device__ __forceinline__ void dma16_buf(uint32_t voff, buffer_rsrc r, uint32_t soff, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "s"(lds_base)
+               : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 template <int N>

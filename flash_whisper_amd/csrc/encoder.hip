@@ -760,10 +760,12 @@ __global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(GemmArgs g) {
 #endif
 static_assert(FW_XCD_GROUP == 0 || FW_XCD_GROUP == 1, "FW_XCD_GROUP is a switch (0 or 1)");
 // Picks the XCD rectangle grid that divides the tile grid and moves the fewest bytes into the L2s:
-// A is fetched once per column group (xn), W once per row group (xm).
+// A is fetched once per column group (xn), W once per row group (xm). Convs too where their weights exceed
+// an L2 (3000 -> 1500 x 1280, k = 3840: 27.2 -> 26.6 us, 1280 -> 640: 21.4 -> 19.3 us); with the short k of
+// the first conv the row-major order is faster (1280 rows: 6.8 against 7.0 us).
 void choose_xcd_groups(GemmArgs& g, int bm, int bn = kBN) {
   g.xm = g.xn = 0;
-  if (!FW_XCD_GROUP || g.conv_stride) return;
+  if (!FW_XCD_GROUP || (g.conv_stride && g.k < 1024)) return;
   const int ntm = (g.m + bm - 1) / bm, ntn = g.n / bn;
   double best = 0;
   for (int xm = 1; xm <= 8; xm *= 2) {

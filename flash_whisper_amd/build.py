@@ -32,11 +32,15 @@ COMMON_FLAGS = [
     '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops',
     '-Xarch_host', '-mfma',
 ]
-# The synthetic-weight generator must round identically on host and device: no FMA contraction.
+# A kernel's leading arguments (up to 14 dwords, not structs) arrive in scalar registers with the launch.
+PRELOAD = ['-mllvm', '-amdgpu-kernarg-preload-count=16']
 PER_FILE_FLAGS = {
+    # the synthetic-weight generator must round identically on host and device: no FMA contraction
     'synth.hip': ['-ffp-contract=off'],
     # MFMA results in VGPRs: the attention softmax reads every score and rescales O in place
-    'attention_enc.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    'attention_enc.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', *PRELOAD],
+    'encoder.hip': PRELOAD,
+    'logmel.hip': PRELOAD,
 }
 
 

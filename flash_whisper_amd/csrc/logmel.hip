@@ -223,6 +223,7 @@ __global__ void __launch_bounds__(kFramesPerBlock * 64) logmel_frames_kernel(con
       const int n = 2 * (lane + kB8 * r);
       const float w0 = 0.5f - 0.5f * tw[n].x, w1 = 0.5f - 0.5f * tw[n + 1].x;
       z[r] = make_float2(z[r].x * w0, z[r].y * w1);
+      asm("" : "+v"(z[r].x), "+v"(z[r].y));  // rounded as they are, not fused into the butterfly's first sums
     }
     fft_butterfly<8, 1>(z, zb, tw, lane);
   }

@@ -121,7 +121,10 @@ constexpr bool epi_reads_res(int epi) {
 // inputs, which are one ulp off (the same count as the Numerical Recipes coefficients, which cost
 // two more FMAs and three more scalings per element; the fc1 epilogue is bound by VALU issue).
 // Beyond z = 4.67 the GELU underflows fp16 on the negative side and equals x on the positive side.
-__device__ __forceinline__ float gelu_enc(float x) {
+// The product x Phi(x) is rounded once, to fp16 (v_fma_mixlo_f16; issued as assembly, because whether the
+// compiler picks it or an fp32 product and a conversion, which rounds twice, depends on what stands around it).
+__device__ __forceinline__ _Float16 gelu_enc(_Float16 xh) {
+  const float x = h2f(xh);
   const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.35355339059327376f, 1.0f));
   float q = -0.19670111f;
   q = fmaf(t, q, 0.74583995f);
@@ -132,16 +135,18 @@ __device__ __forceinline__ float gelu_enc(float x) {
   q = fmaf(t, q, 1.46661794f);
   q = fmaf(t, q, -2.82770705f);
   const float c = t * __builtin_amdgcn_exp2f(fmaf(x * x, -0.72134752f, q));  // Phi(-|x|)
-  return x * (x >= 0.0f ? 1.0f - c : c);
+  const float phi = x >= 0.0f ? 1.0f - c : c;
+  _Float16 y;
+  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(y) : "v"(phi), "v"(xh));
+  return y;
 }
 
 // The epilogue's value before its residual / position operand: an fp16 number for the epilogues that read
 // one, so it can be staged as fp16 without a rounding of its own.
 template <int EPI>
 __device__ __forceinline__ float epilogue_pre(float acc, float b, int col, int q_cols) {
+  if constexpr (EPI == FW_EPI_BIAS_GELU || EPI == FW_EPI_BIAS_GELU_POS) return h2f(gelu_enc(f2h(acc + b)));
   float v = round_h(acc + b);
-  if constexpr (EPI == FW_EPI_BIAS_GELU) v = gelu_enc(v);
-  if constexpr (EPI == FW_EPI_BIAS_GELU_POS) v = round_h(gelu_enc(v));
   if constexpr (EPI == FW_EPI_SCALE_Q || EPI == kEpiQkvVt)
     if (col < q_cols) v = v * 0.125f;
   return v;

@@ -39,6 +39,7 @@ PER_FILE_FLAGS = {
     'synth.hip': ['-ffp-contract=off'],
     # MFMA results in VGPRs: the attention softmax reads every score and rescales O in place
     'attention_enc.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', *PRELOAD],
+    'decode.hip': PRELOAD,
     'encoder.hip': PRELOAD,
     'logmel.hip': PRELOAD,
 }

@@ -51,11 +51,35 @@ __global__ void __launch_bounds__(256) embed_kernel(const int64_t* cur, const in
 // NV input vectors (a batch of decoder positions, NV <= kMaxBatch) share every weight row load: vector
 // v reads x / h / h_out at offset v * K and writes out + v * n; its LN or combine prologue is that of
 // a single-vector launch, so each vector's result is bit-identical to NV separate launches.
+//
+// The first 14 dwords of a kernel's arguments arrive in scalar registers with the launch (the build preloads
+// them); a struct is read from the argument segment, a memory round trip before the first request. So the
+// pointers of the first requests come ahead of the structs: p0 .. p3 are the LayerNorm's h, x, gamma and
+// beta, the combine's part_m, part_l, part_acc and len_state, or the plain input; `dims` is 1 for the
+// embedding mode, or the combine's nsplit | heads << 8 | split_keys << 16. One decoder step of 34 launches
+// in a graph 156.0 -> 144.2 us.
 template <int K, int NW, int U, int MODE, int ACT, int NV = 1>
-__global__ void __launch_bounds__(NW * 64) gemv_kernel(const _Float16* __restrict__ xin, LnArgs ln, CombineArgs cb,
+__global__ void __launch_bounds__(NW * 64) gemv_kernel(const void* __restrict__ p0, const void* __restrict__ p1,
+                                                       const void* __restrict__ p2, const void* __restrict__ p3,
                                                        const _Float16* __restrict__ w,
-                                                       const _Float16* __restrict__ bias, _Float16* __restrict__ out,
-                                                       int n) {
+                                                       const _Float16* __restrict__ bias, int n, int dims,
+                                                       _Float16* __restrict__ out, LnArgs ln, CombineArgs cb) {
+  const _Float16* xin = static_cast<const _Float16*>(p0);
+  const bool embed = MODE == kModeLn && dims != 0;
+  if constexpr (MODE == kModeLn) {
+    ln.h = xin;
+    ln.x = static_cast<const _Float16*>(p1);
+    ln.gamma = static_cast<const _Float16*>(p2);
+    ln.beta = static_cast<const _Float16*>(p3);
+  } else if constexpr (MODE == kModeCombine) {
+    cb.part_m = static_cast<const float*>(p0);
+    cb.part_l = static_cast<const float*>(p1);
+    cb.part_acc = static_cast<const float*>(p2);
+    cb.len_state = static_cast<const int64_t*>(p3);
+    cb.nsplit = dims & 255;
+    cb.heads = (dims >> 8) & 255;
+    cb.split_keys = dims >> 16;
+  }
   using RS = RowSplit<K>;
   constexpr int kRowsPerBlock = NW * RS::kRPW * U;
   __shared__ __align__(16) _Float16 y_lds[MODE != kModePlain ? NV * K : 8];
@@ -74,7 +98,7 @@ __global__ void __launch_bounds__(NW * 64) gemv_kernel(const _Float16* __restric
     for (int v = 0; v < NV; ++v) {
       const _Float16* a = ln.h ? ln.h + v * kHidden : nullptr;
       const _Float16* b = ln.x ? ln.x + v * kHidden : nullptr;
-      if (ln.cur) embed_rows(ln.cur, ln.state, ln.embed, ln.pos_embed, ln.vocab, ln.max_pos, &a, &b, v);
+      if (embed) embed_rows(ln.cur, ln.state, ln.embed, ln.pos_embed, ln.vocab, ln.max_pos, &a, &b, v);
       ln_load<NW * 64>(a, b, ln.gamma, ln.beta, lnr[v]);
     }
   } else if constexpr (MODE == kModeCombine) {
@@ -98,9 +122,9 @@ __global__ void __launch_bounds__(NW * 64) gemv_kernel(const _Float16* __restric
   const uint4* xv;
   if constexpr (MODE == kModeLn) {
     if constexpr (NV == 1)
-      ln_finish<NW * 64, true>(lnr[0], ln.cur != nullptr || ln.x != nullptr, ln.h_out, ln.eps, y_lds, red);
+      ln_finish<NW * 64, true>(lnr[0], embed || ln.x != nullptr, ln.h_out, ln.eps, y_lds, red);
     else
-      ln_finish_multi<NW * 64, NV>(lnr, ln.cur != nullptr || ln.x != nullptr, ln.h_out, ln.eps, y_lds, red);
+      ln_finish_multi<NW * 64, NV>(lnr, embed || ln.x != nullptr, ln.h_out, ln.eps, y_lds, red);
     __syncthreads();
     xv = reinterpret_cast<const uint4*>(y_lds);
   } else if constexpr (MODE == kModeCombine) {
@@ -147,7 +171,18 @@ void launch_gemv(const _Float16* x, const LnArgs& ln, const CombineArgs& cb, con
                  _Float16* out, int n, hipStream_t s) {
   constexpr int kRows = NW * RowSplit<K>::kRPW * U;
   const int grid = (n + kRows - 1) / kRows;
-  hipLaunchKernelGGL((gemv_kernel<K, NW, U, MODE, ACT, NV>), dim3(grid), dim3(NW * 64), 0, s, x, ln, cb, w, b, out, n);
+  const void *p0 = x, *p1 = nullptr, *p2 = nullptr, *p3 = nullptr;
+  int dims = 0;
+  if constexpr (MODE == kModeLn) {
+    p0 = ln.h, p1 = ln.x, p2 = ln.gamma, p3 = ln.beta;
+    dims = ln.cur != nullptr;
+  } else if constexpr (MODE == kModeCombine) {
+    static_assert(kMaxCombineSplits < 256 && kMaxCombineHeads < 256, "packed into dims (split_keys <= 256)");
+    p0 = cb.part_m, p1 = cb.part_l, p2 = cb.part_acc, p3 = cb.len_state;
+    dims = cb.nsplit | cb.heads << 8 | cb.split_keys << 16;
+  }
+  hipLaunchKernelGGL((gemv_kernel<K, NW, U, MODE, ACT, NV>), dim3(grid), dim3(NW * 64), 0, s, p0, p1, p2, p3, w, b, n,
+                     dims, out, ln, cb);
 }
 
 // A batch of nv (1..kMaxBatch) vectors, one row group per wave (the batch runs once per clip, for the
@@ -257,10 +292,13 @@ constexpr int kLmRowsIter = kLmNW * 2 * kLmU;  // rows per block iteration
 
 
 template <bool LN>
-__global__ void __launch_bounds__(kLmNW * 64) lm_head_kernel(const _Float16* __restrict__ yin, LnArgs ln,
+__global__ void __launch_bounds__(kLmNW * 64) lm_head_kernel(const _Float16* __restrict__ h,  // y without LN
+                                                             const _Float16* __restrict__ x,
+                                                             const _Float16* __restrict__ gamma,
+                                                             const _Float16* __restrict__ beta,
                                                              const _Float16* __restrict__ w,
                                                              const uint8_t* __restrict__ suppress, int vocab,
-                                                             unsigned long long* best) {
+                                                             float eps, unsigned long long* best) {
   using RS = RowSplit<kHidden>;
   __shared__ __align__(16) _Float16 y_lds[kHidden];
   __shared__ float red[kLmNW];
@@ -287,16 +325,16 @@ __global__ void __launch_bounds__(kLmNW * 64) lm_head_kernel(const _Float16* __r
     }
   };
   LnRegs<kLmNW * 64> lnr;
-  if constexpr (LN) ln_load<kLmNW * 64>(ln.h, ln.x, ln.gamma, ln.beta, lnr);
+  if constexpr (LN) ln_load<kLmNW * 64>(h, x, gamma, beta, lnr);
   uint4 wa[kLmU][RS::kC], wb[kLmU][RS::kC];
   uint32_t sa[kLmU], sb[kLmU];
   load(base_of(0), wa, sa);
 
   if constexpr (LN) {
-    ln_finish<kLmNW * 64>(lnr, ln.x != nullptr, nullptr, ln.eps, y_lds, red);
+    ln_finish<kLmNW * 64>(lnr, x != nullptr, nullptr, eps, y_lds, red);
   } else {
     for (int i = threadIdx.x; i < kHidden / 8; i += blockDim.x)
-      reinterpret_cast<uint4*>(y_lds)[i] = reinterpret_cast<const uint4*>(yin)[i];
+      reinterpret_cast<uint4*>(y_lds)[i] = reinterpret_cast<const uint4*>(h)[i];
   }
   __syncthreads();
   uint4 xr[RS::kC];
@@ -346,7 +384,10 @@ int lm_head_grid(int vocab) {
   return (batches + per - 1) / per;
 }
 
-__global__ void argmax_finalize_kernel(unsigned long long* best, FinArgs fin) { finalize_token(best, fin); }
+__global__ void argmax_finalize_kernel(unsigned long long* best, int64_t* tokens, int64_t* state, int64_t* cur,
+                                       int max_pos) {
+  finalize_token(best, FinArgs{tokens, state, cur, max_pos});
+}
 
 // ------------------------------------------------------------------------------------------
 // LM head with an int8 pre-pass: the packed winner of lm_head_kernel, bit for bit, from about half
@@ -406,11 +447,14 @@ __global__ void __launch_bounds__(256) lm_q8_pack_kernel(const _Float16* __restr
 }
 
 template <bool LN>
-__global__ void __launch_bounds__(kLmNW * 64) lm_head_q8_kernel(const _Float16* __restrict__ yin, LnArgs ln,
-                                                                const _Float16* __restrict__ w,
+__global__ void __launch_bounds__(kLmNW * 64) lm_head_q8_kernel(const _Float16* __restrict__ h,
+                                                                const _Float16* __restrict__ x,
+                                                                const _Float16* __restrict__ gamma,
+                                                                const _Float16* __restrict__ beta,
                                                                 const int8_t* __restrict__ wq,
-                                                                const float2* __restrict__ meta,
-                                                                const uint8_t* __restrict__ suppress, int vocab,
+                                                                const float2* __restrict__ meta, int vocab, float eps,
+                                                                const _Float16* __restrict__ w,
+                                                                const uint8_t* __restrict__ suppress,
                                                                 unsigned long long* best) {
   __shared__ __align__(16) _Float16 y_lds[kHidden];
   __shared__ __align__(16) int8_t yhi[kHidden];
@@ -440,7 +484,7 @@ __global__ void __launch_bounds__(kLmNW * 64) lm_head_q8_kernel(const _Float16* 
     b.sp = suppress[row];
   };
   LnRegs<kNT> lnr;
-  if constexpr (LN) ln_load<kNT>(ln.h, ln.x, ln.gamma, ln.beta, lnr);
+  if constexpr (LN) ln_load<kNT>(h, x, gamma, beta, lnr);
   if (tid == 0) ncand = 0;
   // The first batch is requested before the LayerNorm, the second after it, the other two as soon as a
   // register buffer frees up. About one 82 KB batch per CU in flight streams faster than more: with
@@ -450,10 +494,10 @@ __global__ void __launch_bounds__(kLmNW * 64) lm_head_q8_kernel(const _Float16* 
   load(base_of(0), ba);
 
   if constexpr (LN) {
-    ln_finish<kNT, true>(lnr, ln.x != nullptr, nullptr, ln.eps, y_lds, red);  // thread tid owns pair tid
+    ln_finish<kNT, true>(lnr, x != nullptr, nullptr, eps, y_lds, red);  // thread tid owns pair tid
   } else {
     for (int i = tid; i < kHidden / 8; i += kNT)
-      reinterpret_cast<uint4*>(y_lds)[i] = reinterpret_cast<const uint4*>(yin)[i];
+      reinterpret_cast<uint4*>(y_lds)[i] = reinterpret_cast<const uint4*>(h)[i];
     __syncthreads();
   }
   load(base_of(1), bb);
@@ -575,12 +619,24 @@ int lm_head_q8_grid(int vocab) {
 }
 
 
+// The split kernel's preloaded arguments (14 dwords, see gemv_kernel), ahead of the struct. It runs inside
+// graphs; the ops called one by one are bound by the host, which pays for every argument (9 arguments
+// instead of 1 made decode_attention 0.3 us a call slower), and keep the struct alone.
+#define FW_ATTN_PARAMS                                                                                              \
+  const _Float16 *q_, _Float16 *k_, _Float16 *v_, const _Float16 *k_new_, const _Float16 *v_new_,                   \
+      const int64_t *len_state_, int max_len_, int split_keys_, AttnArgs a
+#define FW_ATTN_ARGS(a) a.q, a.k, a.v, a.k_new, a.v_new, a.len_state, a.max_len, a.split_keys, a
+#define FW_ATTN_TAKE_PARAMS()                                                                    \
+  a.q = q_, a.k = k_, a.v = v_, a.k_new = k_new_, a.v_new = v_new_, a.len_state = len_state_,    \
+  a.max_len = max_len_, a.split_keys = split_keys_
+
 // BATCH: a batch of queries (grid.z, the prompt) takes the fresh K/V rows of the batch's earlier
 // queries straight from k_new / v_new: their cache rows are written by other blocks of the same
 // launch, so a cache row at or past the batch's first position is never trusted. The single-query
 // instantiation carries none of this code.
 template <int MAXP, bool BATCH, int NW = 4>
-__global__ void __launch_bounds__(NW * 64) attn_split_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(NW * 64) attn_split_kernel(FW_ATTN_PARAMS) {
+  FW_ATTN_TAKE_PARAMS();
   __shared__ float wm[NW], wl[NW];
   __shared__ float wacc[NW][kHeadDim];
   const int split = blockIdx.x, head = blockIdx.y, nsplit = gridDim.x, qv = BATCH ? blockIdx.z : 0;
@@ -658,18 +714,18 @@ int launch_attn_split(const AttnArgs& a, int nsplit, int heads, hipStream_t s, i
   constexpr int kP256 = FW_ATTN256_P, kW256 = 32 / FW_ATTN256_P;
   if (nq == 1) {
     if (a.split_keys <= 64)
-      hipLaunchKernelGGL((attn_split_kernel<2, false>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<2, false>), grid, dim3(256), 0, s, FW_ATTN_ARGS(a));
     else if (a.split_keys <= 128)
-      hipLaunchKernelGGL((attn_split_kernel<4, false>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<4, false>), grid, dim3(256), 0, s, FW_ATTN_ARGS(a));
     else
-      hipLaunchKernelGGL((attn_split_kernel<kP256, false, kW256>), grid, dim3(kW256 * 64), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<kP256, false, kW256>), grid, dim3(kW256 * 64), 0, s, FW_ATTN_ARGS(a));
   } else {
     if (a.split_keys <= 64)
-      hipLaunchKernelGGL((attn_split_kernel<2, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<2, true>), grid, dim3(256), 0, s, FW_ATTN_ARGS(a));
     else if (a.split_keys <= 128)
-      hipLaunchKernelGGL((attn_split_kernel<4, true>), grid, dim3(256), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<4, true>), grid, dim3(256), 0, s, FW_ATTN_ARGS(a));
     else
-      hipLaunchKernelGGL((attn_split_kernel<kP256, true, kW256>), grid, dim3(kW256 * 64), 0, s, a);
+      hipLaunchKernelGGL((attn_split_kernel<kP256, true, kW256>), grid, dim3(kW256 * 64), 0, s, FW_ATTN_ARGS(a));
   }
   return fw_check_launch("attention split");
 }
@@ -679,11 +735,12 @@ int launch_attn_split(const AttnArgs& a, int nsplit, int heads, hipStream_t s, i
 // 448-key cache were 7 round trips to L2 in a row (4.6 us a launch for 20 waves of work).
 constexpr int kCombineBatch = 8;
 
-__global__ void __launch_bounds__(64) attn_combine_kernel(AttnArgs a, int nsplit) {
+__global__ void __launch_bounds__(64) attn_combine_kernel(const float* part_m, const float* part_l,
+                                                          const float* part_acc, _Float16* out, int nsplit) {
   const int head = blockIdx.x, d = threadIdx.x;
-  const float* pm = a.part_m + head * nsplit;
-  const float* pl = a.part_l + head * nsplit;
-  const float* pa = a.part_acc + static_cast<size_t>(head) * nsplit * kHeadDim;
+  const float* pm = part_m + head * nsplit;
+  const float* pl = part_l + head * nsplit;
+  const float* pa = part_acc + static_cast<size_t>(head) * nsplit * kHeadDim;
   float m = -INFINITY;
   for (int s0 = 0; s0 < nsplit; s0 += kCombineBatch) {
     float v[kCombineBatch];
@@ -710,7 +767,7 @@ __global__ void __launch_bounds__(64) attn_combine_kernel(AttnArgs a, int nsplit
       den = live ? fmaf(vl[i], wgt, den) : den;
     }
   }
-  a.out[head * kHeadDim + d] = f2h(num / den);
+  out[head * kHeadDim + d] = f2h(num / den);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -819,7 +876,8 @@ int launch_decode_attention(const AttnArgs& a, int nsplit, int heads, hipStream_
   }
   const int rc = launch_attn_split(a, nsplit, heads, s);
   if (rc != FW_OK) return rc;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(heads), dim3(kHeadDim), 0, s, a, nsplit);
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(heads), dim3(kHeadDim), 0, s, a.part_m, a.part_l, a.part_acc, a.out,
+                     nsplit);
   return fw_check_launch("decode_attention combine");
 }
 
@@ -957,7 +1015,7 @@ extern "C" int fw_lm_head_argmax(const void* y, const void* w, const uint8_t* su
   FW_REQUIRE(aligned16(y) && aligned16(w), "lm_head_argmax: y and w must be 16-byte aligned");
   const int grid = lm_head_grid(vocab);
   hipLaunchKernelGGL(lm_head_kernel<false>, dim3(grid), dim3(kLmNW * 64), 0, stream, static_cast<const _Float16*>(y),
-                     LnArgs{}, static_cast<const _Float16*>(w), suppress, vocab,
+                     nullptr, nullptr, nullptr, static_cast<const _Float16*>(w), suppress, vocab, 0.f,
                      reinterpret_cast<unsigned long long*>(best));
   return fw_check_launch("lm_head_argmax");
 }
@@ -976,13 +1034,14 @@ extern "C" int fw_lm_head_argmax_fused(const void* h, const void* x, const void*
   LnArgs ln{static_cast<const _Float16*>(h), static_cast<const _Float16*>(x), nullptr,
             static_cast<const _Float16*>(gamma), static_cast<const _Float16*>(beta), eps, nullptr, nullptr,
             nullptr, nullptr, 0, 0};
-  hipLaunchKernelGGL(lm_head_kernel<true>, dim3(grid), dim3(kLmNW * 64), 0, stream, nullptr, ln,
-                     static_cast<const _Float16*>(w), suppress, vocab, reinterpret_cast<unsigned long long*>(best));
+  hipLaunchKernelGGL(lm_head_kernel<true>, dim3(grid), dim3(kLmNW * 64), 0, stream, ln.h, ln.x, ln.gamma, ln.beta,
+                     static_cast<const _Float16*>(w), suppress, vocab, ln.eps,
+                     reinterpret_cast<unsigned long long*>(best));
   int rc = fw_check_launch("lm_head_argmax_fused");
   if (rc != FW_OK || !finalize) return rc;
   FinArgs fin{tokens, state, cur, max_pos};
   hipLaunchKernelGGL(argmax_finalize_kernel, dim3(1), dim3(1), 0, stream, reinterpret_cast<unsigned long long*>(best),
-                     fin);
+                     fin.tokens, fin.state, fin.cur, fin.max_pos);
   return fw_check_launch("lm_head_argmax_fused finalize");
 }
 
@@ -1010,15 +1069,14 @@ extern "C" int fw_lm_head_argmax_q8(const void* h, const void* x, const void* ga
   LnArgs ln{static_cast<const _Float16*>(h), static_cast<const _Float16*>(x), nullptr,
             static_cast<const _Float16*>(gamma), static_cast<const _Float16*>(beta), eps, nullptr, nullptr,
             nullptr, nullptr, 0, 0};
-  hipLaunchKernelGGL(lm_head_q8_kernel<true>, dim3(lm_head_q8_grid(vocab)), dim3(kLmNW * 64), 0, stream, nullptr, ln,
-                     static_cast<const _Float16*>(w), static_cast<const int8_t*>(wq),
-                     reinterpret_cast<const float2*>(meta), suppress, vocab,
-                     reinterpret_cast<unsigned long long*>(best));
+  hipLaunchKernelGGL(lm_head_q8_kernel<true>, dim3(lm_head_q8_grid(vocab)), dim3(kLmNW * 64), 0, stream, ln.h, ln.x,
+                     ln.gamma, ln.beta, static_cast<const int8_t*>(wq), reinterpret_cast<const float2*>(meta), vocab,
+                     ln.eps, static_cast<const _Float16*>(w), suppress, reinterpret_cast<unsigned long long*>(best));
   int rc = fw_check_launch("lm_head_argmax_q8");
   if (rc != FW_OK || !finalize) return rc;
   FinArgs fin{tokens, state, cur, max_pos};
   hipLaunchKernelGGL(argmax_finalize_kernel, dim3(1), dim3(1), 0, stream, reinterpret_cast<unsigned long long*>(best),
-                     fin);
+                     fin.tokens, fin.state, fin.cur, fin.max_pos);
   return fw_check_launch("lm_head_argmax_q8 finalize");
 }
 
@@ -1028,7 +1086,7 @@ extern "C" int fw_argmax_finalize(uint64_t* best, int64_t* tokens, int64_t* stat
   FW_REQUIRE(max_pos > 0, "max_pos must be positive");
   FinArgs fin{tokens, state, cur, max_pos};
   hipLaunchKernelGGL(argmax_finalize_kernel, dim3(1), dim3(1), 0, stream, reinterpret_cast<unsigned long long*>(best),
-                     fin);
+                     fin.tokens, fin.state, fin.cur, fin.max_pos);
   return fw_check_launch("argmax_finalize");
 }
 

@@ -940,8 +940,10 @@ int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
 // Row LayerNorm over 1280 columns: 32 lanes per row (5 x 16-byte chunks each), kLnRows = kLnThreads / 32 rows per block.
 // ------------------------------------------------------------------------------------------
 constexpr int kLnC = kHidden / 8 / 32;  // 16-byte fp16 chunks per lane of a row
+// One wave (two rows) a block: 251 rows make 126 blocks instead of 32 (the encoder over 251 frames 295.6 ->
+// 291.2 us, over 1500 frames 4292 -> 4284 us; 128 threads 292.1 and 4315 us).
 #ifndef FW_LN_THREADS
-#define FW_LN_THREADS 256
+#define FW_LN_THREADS 64
 #endif
 constexpr int kLnThreads = FW_LN_THREADS;  // threads per row-LayerNorm block: 32 lanes per row
 constexpr int kLnRows = kLnThreads / 32;

@@ -592,6 +592,116 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(FW_GEMM
   }
 }
 
+// ---- 256 x 256 tiles ------------------------------------------------------------------------------
+// The cross K/V of 3 or 4 decoder layers: products so wide that 256 x 128 tiles take two passes over the
+// CUs. 2 x 4 waves of 128 x 64, a ring of two 64 KB stages; a stage's operands are read 16 of k at a time,
+// double-buffered in registers, and the last 16 are multiplied behind the barrier of the next stage, while
+// its first are read. A tile moves 2/3 of the bytes per product of a 256 x 128 one, which matters where
+// power sets the clock (about 1.9 GHz in these products). 1500 x 10240 x 1280: 47.8 -> 41.1 us a call.
+constexpr int kWideWaves = 8, kWide = 256, kWideStage = 2 * kWide * 128;
+constexpr int kWideRowH = kWide + 8;  // halves per staged output row
+constexpr int kWideLds = kWide * kWideRowH * 2 > 2 * kWideStage ? kWide * kWideRowH * 2 : 2 * kWideStage;
+
+__global__ void __launch_bounds__(kWideWaves * 64) gemm_wide_kv_kernel(FW_GEMM_PARAMS) {
+  FW_GEMM_TAKE_PARAMS();
+  constexpr int kTM = 4, kTN = 2, kCopies = kWide / 8 / kWideWaves;  // copies per wave of each operand
+  __shared__ __align__(1024) u32x4 lds[kWideLds / 16];
+  int m0, n0;
+  tile_origin<kWide, kWide>(g, m0, n0);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 2) * 128, wn = (wave & 3) * 64, lr = lane & 31, lg = lane >> 5;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  uint32_t aoff[kCopies], woff[kCopies];
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) {
+    const int row = (wave * kCopies + i) * 8 + (lane >> 3), chunk = swz_slot(row, lane & 7) * 8;
+    aoff[i] = static_cast<uint32_t>((static_cast<size_t>(min(m0 + row, g.m - 1)) * g.lda + chunk) * 2);
+    woff[i] = static_cast<uint32_t>((static_cast<size_t>(n0 + row) * g.ldw + chunk) * 2);
+  }
+  auto issue = [&](int kt) {
+    const uint32_t dst = lds0 + (kt & 1) * kWideStage + wave * kCopies * 1024;
+    const size_t kb = static_cast<size_t>(kt) * (kBK * 2);
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) dma16_s(aoff[i], reinterpret_cast<const char*>(g.a) + kb, dst + i * 1024);
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i)
+      dma16_s(woff[i], reinterpret_cast<const char*>(g.w) + kb, dst + kWide * 128 + i * 1024);
+  };
+  const FragOffsets fo = frag_offsets<kWide>(wm, wn, lr, lg);
+  struct Step {
+    h8v a[kTM], b[kTN];
+  };
+  auto read = [&](int kt, int s, Step& f) {
+    const char* stage = reinterpret_cast<const char*>(lds) + (kt & 1) * kWideStage;
+#pragma unroll
+    for (int i = 0; i < kTM; ++i) f.a[i] = *reinterpret_cast<const h8v*>(stage + fo.a[s] + 4096 * i);
+#pragma unroll
+    for (int j = 0; j < kTN; ++j) f.b[j] = *reinterpret_cast<const h8v*>(stage + fo.b[s] + 4096 * j);
+  };
+  f16v acc[kTM][kTN];
+#pragma unroll
+  for (int i = 0; i < kTM; ++i)
+#pragma unroll
+    for (int j = 0; j < kTN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  auto multiply = [&](const Step& f) {
+#pragma unroll
+    for (int i = 0; i < kTM; ++i)
+#pragma unroll
+      for (int j = 0; j < kTN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
+  };
+  const int kt_n = g.k / kBK;
+  // stage kt has landed and every wave sees it; every wave has read stage kt - 1, whose slot is refilled
+  auto enter = [&](int kt) {
+    wait_vmcnt<0>();
+    lds_barrier();
+    if (kt + 1 < kt_n) issue(kt + 1);
+  };
+  Step f0, f1;
+  issue(0);
+  enter(0);
+  read(0, 0, f0);
+  for (int kt = 0; kt < kt_n; ++kt) {
+    read(kt, 1, f1);
+    multiply(f0);
+    read(kt, 2, f0);
+    multiply(f1);
+    read(kt, 3, f1);
+    multiply(f0);
+    if (kt + 1 < kt_n) {
+      enter(kt + 1);
+      read(kt + 1, 0, f0);
+    }
+    multiply(f1);
+  }
+  __syncthreads();  // every wave has read its last operands
+  _Float16* t = reinterpret_cast<_Float16*>(lds);
+#pragma unroll
+  for (int j = 0; j < kTN; ++j)
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      const int cl = wn + 32 * j + 8 * rq + 4 * lg;  // columns cl .. cl + 3 of the tile
+      h4u bb = {};
+      if (g.bias) bb = *reinterpret_cast<const h4u*>(g.bias + n0 + cl);
+#pragma unroll
+      for (int i = 0; i < kTM; ++i) {
+        h4v o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = f2h(acc[i][j][4 * rq + e] + h2f(bb[e]));
+        *reinterpret_cast<h4v*>(t + (wm + 32 * i + lr) * kWideRowH + cl) = o;
+      }
+    }
+  __syncthreads();
+#pragma unroll 4
+  for (int c = tid; c < kWide * (kWide / 8); c += kWideWaves * 64) {
+    const int rl = c / (kWide / 8), cl = c % (kWide / 8) * 8, row = m0 + rl, col = n0 + cl;
+    if (row < g.m)
+      *reinterpret_cast<h8u*>(g.out + (static_cast<size_t>(col >> 6) * g.t_len + row) * 64 + (col & 63)) =
+          *reinterpret_cast<const h8v*>(t + rl * kWideRowH + cl);
+  }
+}
+
 // ---- k-sliced GEMM for few rows ----------------------------------------------------------------
 // out = epilogue(A W^T) where the tiles of gemm_dma_kernel would leave most CUs idle. A block's kKsWaves
 // waves all compute the whole TM x TN tile, wave w over the 64-wide k stages w, w + kKsWaves, ...: each
@@ -871,13 +981,14 @@ int launch_ks(GemmArgs g, int epi, hipStream_t s) {
 //   (1200, 5120, 1280) 128x128 34.3 (2), 192x128 38.0 (2), 256x128 30.4
 //   (251, 1280, 2 x 2560) 64x32 19.4 (2), 64x64 15.1, 96x64 17.7, 128x128 28.4
 //   (400, 1280, 2 x 2560) 64x64 26.1 (2), 96x64 17.6, 128x128 23.1
-enum Tile { kD256, kD192, kD128, kD64, kS96x64, kS64x64, kS64x32, kS32x32, kTiles };
+enum Tile { kD256, kD192, kD128, kD64, kS96x64, kS64x64, kS64x32, kS32x32, kWide256, kTiles };
 struct TileCost {
   int rows, cols;
   float per_stage;  // us per 64-wide k stage and pass
 };
 constexpr TileCost kTileCost[kTiles] = {{256, 128, 1.15f}, {192, 128, 0.85f}, {128, 128, 0.62f}, {64, 128, 0.42f},
-                                        {96, 64, 0.43f},   {64, 64, 0.28f},   {64, 32, 0.18f},   {32, 32, 0.11f}};
+                                        {96, 64, 0.43f},   {64, 64, 0.28f},   {64, 32, 0.18f},   {32, 32, 0.11f},
+                                        {kWide, kWide, 1.55f}};
 constexpr float kPassUs = 4.f;
 constexpr int kCus = 256;
 
@@ -902,7 +1013,8 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
 
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
-  switch (choose_tile(g, [](Tile) { return true; })) {
+  const bool wide = epi == kEpiCrossKV && g.n % kWide == 0;  // the one epilogue that the wide tiles have
+  switch (choose_tile(g, [&](Tile t) { return t != kWide256 || wide; })) {
     case kD256: return launch_dma<256, kNoConv>(g, epi, s);
     case kD192: return launch_dma<192, kNoConv>(g, epi, s);
     case kD64: return launch_dma<64, kNoConv>(g, epi, s);
@@ -910,6 +1022,13 @@ int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
     case kS64x64: return launch_ks<64, 64, false>(g, epi, s);
     case kS64x32: return launch_ks<64, 32, false>(g, epi, s);
     case kS32x32: return launch_ks<32, 32, false>(g, epi, s);
+    case kWide256: {
+      GemmArgs w = g;
+      choose_xcd_groups(w, kWide, kWide);
+      hipLaunchKernelGGL(gemm_wide_kv_kernel, dim3((g.n / kWide) * ((g.m + kWide - 1) / kWide)), dim3(kWideWaves * 64), 0, s,
+                         FW_GEMM_ARGS(w));
+      return fw_check_launch("gemm");
+    }
     default: return launch_dma<128, kNoConv>(g, epi, s);
   }
 }
@@ -920,7 +1039,7 @@ int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
 // register-staged gather, 10.3 for a 2-deep ring and 10.1 for 128-row tiles; 1000 rows: 6.7, 10.5, 7.8, 9.4).
 int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
   if (!conv_offsets_fit(g) || !copy_offsets_fit(g)) return launch_dma<128, kConvAny>(g, epi, s);
-  switch (choose_tile(g, [&](Tile t) { return t >= kD128; })) {
+  switch (choose_tile(g, [&](Tile t) { return t >= kD128 && t != kWide256; })) {
     case kS64x64: return launch_ks<64, 64, true>(g, epi, s);
     case kS64x32: return launch_ks<64, 32, true>(g, epi, s);
     case kS32x32: return launch_ks<32, 32, true>(g, epi, s);
@@ -1153,7 +1272,7 @@ extern "C" int fw_gemm_splitk(const void* a, int lda, const void* w, int ldw, fl
   g.splits = splits;
   g.part = part;
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm_splitk: each operand must span less than 4 GiB");
-  switch (choose_tile(g, [](Tile t) { return t == kD128 || t > kD64; })) {
+  switch (choose_tile(g, [](Tile t) { return t == kD128 || (t > kD64 && t != kWide256); })) {
     case kS96x64: return launch_ks<96, 64, false>(g, kEpiPartial, stream);
     case kS64x64: return launch_ks<64, 64, false>(g, kEpiPartial, stream);
     case kS64x32: return launch_ks<64, 32, false>(g, kEpiPartial, stream);

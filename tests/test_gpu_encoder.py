@@ -261,6 +261,22 @@ def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m):
     assert torch.equal(vt, vt_ref)
 
 
+@pytest.mark.parametrize('t,layers', [(1500, 4), (1025, 3), (1281, 4)])
+def test_cross_kv_wide_tiles_match_gemm(ext, hip_device, t, layers):
+    """Sizes that take the 256 x 256 tiles (whole and partial last row tiles): the bits of the plain product,
+    whose tiles add the same terms in the same order, in the cache layout."""
+    rng = np.random.default_rng(t)
+    enc = h16(rng.standard_normal((t, 1280)), hip_device)
+    n = layers * 2 * 1280
+    w = torch.randn(n, 1280, device=hip_device, generator=torch.Generator(device=hip_device).manual_seed(t)).mul_(0.02).half()
+    b = h16(0.02 * rng.standard_normal(n), hip_device)
+    ref = torch.empty(t, n, dtype=torch.float16, device=hip_device)
+    ext.gemm(enc, w, b, ref, 0)
+    out = torch.full((layers, 2, 20, t, 64), float('nan'), dtype=torch.float16, device=hip_device)
+    ext.cross_kv(enc, w, b, out)
+    assert torch.equal(out, ref.view(t, layers, 2, 20, 64).permute(1, 2, 3, 0, 4))
+
+
 def test_cross_kv_layout(ext, hip_device):
     from flash_whisper_amd.config import TURBO
 

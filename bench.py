@@ -26,8 +26,8 @@ graph's stream; with ``--fp16-lm-head`` the step is not one launch and ``rooflin
 ``clips`` holds the reference's clip-length rows: 5 s and 15 s seeded clips, 20 transcribes each with
 the token budget scaled to the clip (37 and 112), and the 30 s timed transcribes; E2E and TTFT median
 and p90. ``configs`` times the path's per-config units: standalone (each over rotating buffers of more
-than 300 MB so every call streams from HBM: the log-mel front end, the 34-launch step's split-K self
-attention at L in {1, 64, 224, 448}, and its cross attention over 1500 frames + LN/GELU MLP), and
+than 300 MB so every call streams from HBM: the log-mel front end, decode_attention's self
+attention at L in {1, 64, 224, 448}, and the cross attention over 1500 frames + LN/GELU MLP), and
 ``in_kernel``: the same units as phases of the persistent step, from its profiling build. Every row
 names its code path. ``cpu_baseline`` times the reference's PyTorch path in fp32 on this host's cores
 (oracle.torch_cpu; 5 end-to-end transcribes and 50 reps per config unit) and runs the numpy oracle once
@@ -273,7 +273,7 @@ def config_rows(model, reps):
     rows['log_mel']['code_path'] = 'logmel_frames_kernel + logmel_finalize_kernel, as transcribe runs them'
     del waves, outs, ws
 
-    # config 2: split-K self attention (split + combine, the reference op) over an fp16 K/V cache
+    # config 2: split-K self attention (decode_attention, the reference op) over an fp16 K/V cache
     heads, hd, max_pos = d.heads, d.head_dim, d.max_pos
     per = 2 * heads * max_pos * hd * 2
     n = -(-ROTATE_BYTES // per)
@@ -286,10 +286,10 @@ def config_rows(model, reps):
         state = torch.tensor([length - 1, 0], dtype=torch.long, device=dev)
         us = graph_time_us(lambda i: ext.decode_attention(q, caches[i % n][0], caches[i % n][1], out, state, kn, vn,
                                                           pm, pl, pa, hd ** -0.5), reps)
-        self_rows[f'L{length}'] = _row(us, 5120 * length + 15360, 2,
+        self_rows[f'L{length}'] = _row(us, 5120 * length + 15360, 1,
                                        f'{n} distinct [20, 448, 64] K/V caches, {reps} calls per graph')
-    self_rows['code_path'] = ('attn_split_kernel + attn_combine_kernel (decode_attention: the 34-launch step\'s '
-                              'kernels, the reference op\'s granularity); the product\'s in-kernel phase is '
+    self_rows['code_path'] = ('attn_direct_kernel (decode_attention in one launch: caches of up to 512 keys, the '
+                              'reference op\'s granularity); the product\'s in-kernel phase is '
                               'in_kernel.self_attention')
     rows['self_attention'] = self_rows
     del caches

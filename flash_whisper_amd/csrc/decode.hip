@@ -201,9 +201,13 @@ void launch_gemv_batch(int nv, const _Float16* x, const LnArgs& ln, const Combin
 }
 
 // Block shapes of the decode GEMVs (waves per block, row groups per wave), measured on MI355X over the
-// whole decoder step (alternating runs of each shape on one device): large blocks (8-12 waves, 54-160
-// blocks) beat one small block per CU because the prologue (LayerNorm or split-K combine) is repeated
-// per block and its latency is the critical path; 4- and 16-wave blocks were slower everywhere.
+// whole decoder step (alternating runs of each shape on one device): where there is a prologue (LayerNorm
+// or split-K combine), large blocks (8 waves, 80-240 blocks) beat one small block per CU because it is
+// repeated per block and its latency is the critical path; 4- and 16-wave blocks were slower. fc2 has no
+// prologue: 5 waves give its 1280 rows one block on each CU. With the first arguments preloaded, the
+// 34-launch step in us, three rounds in turn: fc2 8 waves and combine 12 144.5 / 144.6 / 144.8, fc2 5
+// 142.8 / 142.3 / 143.0, combine 8 143.1 / 142.6 / 142.7, both 141.9 / 141.3 / 141.0. Others: fc2 10 147,
+// 16 152; combine 10 146, 16 148, with fc2 5: 6 142.1, 5 146.2; fc1 in one row group 147, q/k/v in two 147.
 #ifndef FW_G5120_NW
 #define FW_G5120_NW 8  // LN + fc1 (5120 rows): 32 rows per block
 #endif
@@ -220,13 +224,13 @@ void launch_gemv_batch(int nv, const _Float16* x, const LnArgs& ln, const Combin
 #define FW_G1280_NW 8  // LN + cross q (1280 rows): 16 rows per block
 #endif
 #ifndef FW_GK5120_NW
-#define FW_GK5120_NW 8  // fc2 (K = 5120): 8 rows per block
+#define FW_GK5120_NW 5  // fc2 (K = 5120): 5 rows per block
 #endif
 #ifndef FW_GK5120_U
 #define FW_GK5120_U 1
 #endif
 #ifndef FW_CMB_NW
-#define FW_CMB_NW 12  // combine + out projection: 24 rows per block
+#define FW_CMB_NW 8  // combine + out projection: 16 rows per block
 #endif
 // Block shapes are whole blocks within the 1024-thread launch bound with at least one row group per
 // wave; any such shape computes the same rows (each row's lane split and order depend on K only).

@@ -83,6 +83,34 @@ def test_gemv(ext, hip_device, n, k, act):
     close_rel(np32(out), ref)
 
 
+@pytest.mark.parametrize('n', [1, 4, 5, 6, 15, 16, 17, 1279, 1281])
+def test_gemv_block_edges(ext, hip_device, n):
+    """Row counts around the blocks' 5 rows (k = 5120) and 16 rows (the combine + out projection): every
+    row as in one call over more rows, bit for bit, and nothing written past the last."""
+    from flash_whisper_amd.selftest import workspace
+
+    dev, heads, rows = hip_device, 20, 1296
+    rng = np.random.default_rng(n)
+    ws = workspace(heads, 1)
+    q, k, v = _attn_inputs(rng, heads, 64)
+    ext.attention_split(h16(q, dev), h16(k, dev), h16(v, dev), None, None, None, *ws, 0.125, split_keys=64)
+    x = h16(rng.standard_normal(5120), dev)
+
+    def fc2(w, b, out):
+        ext.gemv(x, w, b, out)
+
+    def attn_out(w, b, out):
+        ext.attn_out_gemv(*ws, None, heads, 64, w, b, out, split_keys=64)
+
+    for op, kk in ((fc2, 5120), (attn_out, 1280)):
+        w, b = h16(0.02 * rng.standard_normal((rows, kk)), dev), h16(rng.standard_normal(rows), dev)
+        full = torch.empty(rows, dtype=torch.float16, device=dev)
+        out = torch.full_like(full, 7.)
+        op(w, b, full)
+        op(w[:n], b[:n], out[:n])
+        assert torch.equal(out[:n], full[:n]) and bool((out[n:] == 7).all())
+
+
 @pytest.mark.parametrize('n,act,embed', [(3840, 0, False), (1280, 0, False), (5120, 1, False), (3840, 0, True)])
 def test_ln_gemv(ext, hip_device, n, act, embed):
     from oracle.common import f16, gelu

@@ -24,17 +24,19 @@ __device__ __forceinline__ int swz(int row, int chunk) { return row * 8 + swz_sl
 // a wave instruction fills 1 KB = 8 rows of 128 bytes. The XOR swizzle is applied on the source
 // side: lane l fills LDS row r0 + l / 8, slot l % 8, so it fetches chunk swz_slot(row, l % 8).
 // The copies are issued from inline assembly: the compiler then does not guard every LDS read with
-// a wait for all outstanding copies, and the pipeline depth is set by the explicit vmcnt waits.
+// a wait for all outstanding copies, and the pipeline depth is set by the explicit vmcnt waits. A scalar
+// write of M0 needs one wait state before an LDS copy reads it, which the hardware does not insert and the
+// compiler does not look for inside an asm block: hence the s_nop.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_base) : "memory", "m0");
 }
 // The same copy from a wave-uniform base (scalar registers) plus a 32-bit per-lane byte offset. A
 // loop that walks the base (one k stage after another) then needs no per-copy address arithmetic in
 // the vector unit: the offsets stay in registers and only the scalar base moves.
 __device__ __forceinline__ void dma16_s(uint32_t voff, const void* sbase, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_base)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_base)
                : "memory", "m0");
 }
 // The same copy through a raw buffer: a lane whose offset lies past the buffer's end fills its chunk with
@@ -47,7 +49,8 @@ __device__ __forceinline__ buffer_rsrc make_rsrc(const void* base, uint32_t byte
 }
 constexpr uint32_t kPastEnd = 0x80000000u;  // an offset past the end of any buffer of less than 2 GiB
 __device__ __forceinline__ void dma16_buf(uint32_t voff, buffer_rsrc r, uint32_t soff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff), "s"(lds_base)
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(r), "s"(soff),
+               "s"(lds_base)
                : "memory", "m0");
 }
 #pragma clang diagnostic pop

@@ -173,3 +173,13 @@ def test_product_filterbank_matches_transformers():
 
     z = np.load(GOLDEN / 'hf_logmel.npz')
     np.testing.assert_allclose(mel_filters(), z['mel_filters'].astype(np.float32), rtol=1e-6, atol=1e-9)
+
+
+def test_lds_copies_wait_after_m0():
+    """A scalar write of M0 and an LDS copy that reads it stand one wait state apart; in inline assembly only the
+    source can put it there."""
+    asm = [s for p in sorted((ROOT / 'flash_whisper_amd' / 'csrc').iterdir())
+           for s in re.findall(r'asm volatile\("([^"]*\bm0,[^"]*)"', p.read_text())]
+    assert len(asm) >= 3
+    for s in asm:
+        assert re.match(r's_mov_b32 m0, %\d\\n\\ts_nop 0\\n\\t(global|buffer)_load', s), s

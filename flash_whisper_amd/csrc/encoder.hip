@@ -343,11 +343,15 @@ __device__ __forceinline__ void copy_offsets(const GemmArgs& g, int m0, int n0, 
 // input row early, and a copy's source is again a per-lane offset plus a scalar one. Only row 0 at the
 // first tap and the last input row's successor at the third fall outside x: their lanes' offsets point past
 // the buffer's end there, which reads as zero (3000 -> 1500 x 1280, k = 3840: 29.5 against 31.6 us with the
-// source row worked out, compared and selected for every copy). Buffers of less than 2 GiB only.
+// source row worked out, compared and selected for every copy). Buffers of less than 2 GiB only. The scalar
+// offset, up to the start of the third tap's last stage, is taken from the buffer's length before a lane's
+// offset is compared, so the length is at least three rows: a one-row input would let it run past the end
+// and the difference wrap. Every lane that reads outside x has the offset past the end, whatever the length.
+__host__ __device__ constexpr int64_t conv_buffer_rows(int t_in) { return t_in + int64_t{1} > 3 ? t_in + int64_t{1} : 3; }
 struct ConvSource {
   buffer_rsrc x;
   __device__ __forceinline__ explicit ConvSource(const GemmArgs& g)
-      : x(make_rsrc(g.a - g.c_in, static_cast<uint32_t>(g.t_in + 1) * g.c_in * 2)) {}
+      : x(make_rsrc(g.a - g.c_in, static_cast<uint32_t>(conv_buffer_rows(g.t_in) * g.c_in * 2))) {}
   // this lane's chunk of A row gm, LDS row `row`, slot `slot`: its offset at each tap
   __device__ __forceinline__ static void offsets(const GemmArgs& g, int gm, int row, int slot, uint32_t (&o)[3]) {
     const int r = gm * g.conv_stride;
@@ -359,9 +363,7 @@ struct ConvSource {
     dma16_buf(tap == 0 ? o[0] : tap == 1 ? o[1] : o[2], x, kk * 2, lds_base);
   }
 };
-bool conv_offsets_fit(const GemmArgs& g) {
-  return (static_cast<size_t>(g.t_in) + 1) * g.c_in * 2 < kPastEnd;
-}
+bool conv_offsets_fit(const GemmArgs& g) { return conv_buffer_rows(g.t_in) * g.c_in * 2 < kPastEnd; }
 
 template <int BM, int kNW>
 __device__ __forceinline__ void dma_stage_w(const GemmArgs& g, const CopyOffsets<BM, kNW>& c, int kt, int wave,

@@ -56,8 +56,9 @@ __global__ void __launch_bounds__(256) embed_kernel(const int64_t* cur, const in
 // them); a struct is read from the argument segment, a memory round trip before the first request. So the
 // pointers of the first requests come ahead of the structs: p0 .. p3 are the LayerNorm's h, x, gamma and
 // beta, the combine's part_m, part_l, part_acc and len_state, or the plain input; `dims` is 1 for the
-// embedding mode, or the combine's nsplit | heads << 8 | split_keys << 16. One decoder step of 34 launches
-// in a graph 156.0 -> 144.2 us.
+// embedding mode, or the combine's nsplit | heads << 8 (split_keys, of any size, is read from the struct with
+// max_len: both are needed once the length is there). One decoder step of 34 launches in a graph 156.0 ->
+// 144.2 us.
 template <int K, int NW, int U, int MODE, int ACT, int NV = 1>
 __global__ void __launch_bounds__(NW * 64) gemv_kernel(const void* __restrict__ p0, const void* __restrict__ p1,
                                                        const void* __restrict__ p2, const void* __restrict__ p3,
@@ -77,8 +78,7 @@ __global__ void __launch_bounds__(NW * 64) gemv_kernel(const void* __restrict__ 
     cb.part_acc = static_cast<const float*>(p2);
     cb.len_state = static_cast<const int64_t*>(p3);
     cb.nsplit = dims & 255;
-    cb.heads = (dims >> 8) & 255;
-    cb.split_keys = dims >> 16;
+    cb.heads = dims >> 8;
   }
   using RS = RowSplit<K>;
   constexpr int kRowsPerBlock = NW * RS::kRPW * U;
@@ -177,9 +177,9 @@ void launch_gemv(const _Float16* x, const LnArgs& ln, const CombineArgs& cb, con
     p0 = ln.h, p1 = ln.x, p2 = ln.gamma, p3 = ln.beta;
     dims = ln.cur != nullptr;
   } else if constexpr (MODE == kModeCombine) {
-    static_assert(kMaxCombineSplits < 256 && kMaxCombineHeads < 256, "packed into dims (split_keys <= 256)");
+    static_assert(kMaxCombineSplits < 256, "packed into dims");
     p0 = cb.part_m, p1 = cb.part_l, p2 = cb.part_acc, p3 = cb.len_state;
-    dims = cb.nsplit | cb.heads << 8 | cb.split_keys << 16;
+    dims = cb.nsplit | cb.heads << 8;
   }
   hipLaunchKernelGGL((gemv_kernel<K, NW, U, MODE, ACT, NV>), dim3(grid), dim3(NW * 64), 0, s, p0, p1, p2, p3, w, b, n,
                      dims, out, ln, cb);
@@ -1312,7 +1312,7 @@ static int attn_out_gemv_impl(const float* part_m, const float* part_l, const fl
   FW_REQUIRE(heads * kHeadDim == kHidden, "attn_out_gemv: heads * 64 must be %d", kHidden);
   FW_REQUIRE(max_len > 0 && split_keys >= 8 && n_out > 0, "attn_out_gemv: bad sizes");
   FW_REQUIRE(aligned16(w), "attn_out_gemv: w must be 16-byte aligned");
-  const int nsplit = (max_len + split_keys - 1) / split_keys;
+  const int nsplit = static_cast<int>((max_len + int64_t{split_keys} - 1) / split_keys);
   FW_REQUIRE(nsplit <= kMaxCombineSplits && heads <= kMaxCombineHeads,
              "attn_out_gemv: at most %d splits (got %d) and %d heads", kMaxCombineSplits, nsplit, kMaxCombineHeads);
   FW_REQUIRE(ws_slots >= static_cast<int64_t>(nv) * heads * nsplit, "attn_out_gemv: workspace too small");

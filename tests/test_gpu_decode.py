@@ -222,6 +222,33 @@ def test_decode_attention_one_launch_edges(ext, hip_device, max_len, length, own
     assert np.array_equal(tk.cpu().numpy(), k, equal_nan=True) and np.array_equal(tv.cpu().numpy(), v, equal_nan=True)
 
 
+@pytest.mark.parametrize('split_keys,max_len,pos', [(256, 448, 100), (32760, 40000, 32759), (32768, 40000, 32768),
+                                                    (65535, 448, 447), (65536, 70000, 65536), (1 << 20, 448, 0),
+                                                    (2 ** 31 - 1, 448, 447)])
+@pytest.mark.parametrize('nv', [1, 4])
+def test_attn_out_gemv_wide_splits(ext, hip_device, split_keys, max_len, pos, nv):
+    """Split sizes of any width: the combine takes the splits that hold keys (positions pos .. pos + nv - 1 of a
+    batch, kept below max_len) and nothing of the others, whose partials are NaN here."""
+    dev, heads = hip_device, 20
+    rng = np.random.default_rng(split_keys % 1000)
+    nsplit = -(-max_len // split_keys)
+    m, l = rng.standard_normal((nv, heads, nsplit)), 1 + rng.random((nv, heads, nsplit))
+    acc = rng.standard_normal((nv, heads, nsplit, 64))
+    w, b = np.float16(0.02 * rng.standard_normal((1280, 1280))), np.float16(0.02 * rng.standard_normal(1280))
+    ref = []
+    for i in range(nv):
+        live = min(pos + i, max_len - 1) // split_keys + 1
+        m[i, :, live:] = l[i, :, live:] = acc[i, :, live:] = np.nan
+        e = np.exp(m[i, :, :live] - m[i, :, :live].max(1, keepdims=True))
+        x = np.float16((acc[i, :, :live] * e[..., None]).sum(1) / (l[i, :, :live] * e).sum(1, keepdims=True))
+        ref.append(x.reshape(1280).astype(np.float64) @ w.T.astype(np.float64) + b)
+    ws = [torch.from_numpy(t.astype(np.float32).ravel()).to(dev) for t in (m, l, acc)]
+    out = torch.empty(nv * 1280, dtype=torch.float16, device=dev)
+    ext.attn_out_gemv(*ws, torch.tensor([pos, 0], device=dev), heads, max_len, h16(w, dev), h16(b, dev), out,
+                      split_keys=split_keys, nv=nv)
+    close_rel(np32(out).reshape(nv, 1280), np.array(ref))
+
+
 def _lm_setup(dev, seed=4):
     from flash_whisper_amd import weights
 

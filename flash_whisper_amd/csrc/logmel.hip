@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(kFramesPerBlock * 64) logmel_frames_kernel(con
   __shared__ float2 tw[kNfft];
   __shared__ float2 bufs[kFramesPerBlock][2][kFftBuf];
   __shared__ float pws[kFramesPerBlock][kBins];
-  __shared__ float mw[kRun * kMels];
+  __shared__ __align__(16) float mw[kRun * kMels];  // filled 16 bytes at a time
   __shared__ float tile[kMels][kFramesPerBlock + 1];
   __shared__ float red[kFramesPerBlock];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -29,12 +29,18 @@ WAVE_CHUNK = 240000  # samples per staged chunk of the waveform upload (half of 
 
 
 _F16, _F32, _I64 = torch.float16, torch.float32, torch.int64
-_device, _raw_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+# absent from a torch without GPU support
+_device = getattr(torch._C, '_cuda_getDevice', None)
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)
 
 
 def _stream():
-    """The current stream's handle, without the Stream object torch.cuda.current_stream() makes (1 us)."""
-    return _raw_stream(_device())
+    """The current stream's handle, without the Stream object torch.cuda.current_stream() makes (1 us). Before
+    torch's first GPU call, in a forked child and without GPU support that function is asked: it initialises
+    or raises."""
+    if torch.cuda.is_initialized() and _raw_stream is not None:
+        return _raw_stream(_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):

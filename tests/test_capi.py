@@ -175,6 +175,31 @@ def test_product_filterbank_matches_transformers():
     np.testing.assert_allclose(mel_filters(), z['mel_filters'].astype(np.float32), rtol=1e-6, atol=1e-9)
 
 
+def test_stream_of_a_torch_without_gpu(monkeypatch):
+    """The op module imports where torch has no GPU support, and asking for a stream then raises torch's error."""
+    import importlib.util
+
+    for name in ('_cuda_getDevice', '_cuda_getCurrentRawStream'):
+        monkeypatch.delattr(torch._C, name, raising=False)
+    spec = importlib.util.spec_from_file_location('flash_whisper_amd.ext_without_gpu',
+                                                  ROOT / 'flash_whisper_amd' / 'ext.py')
+    ext = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(ext)
+    if not torch.cuda.is_available():
+        with pytest.raises((RuntimeError, AssertionError)):
+            ext._stream()
+
+
+def test_stream_in_a_forked_child_is_refused(monkeypatch):
+    """A child forked after the first GPU call has no stream: torch says so before anything reaches HIP."""
+    from flash_whisper_amd import ext
+
+    monkeypatch.setattr(torch.cuda, '_initialized', True)
+    monkeypatch.setattr(torch.cuda, '_is_in_bad_fork', lambda: True)
+    with pytest.raises(RuntimeError, match='forked subprocess'):
+        ext._stream()
+
+
 def test_lds_copies_wait_after_m0():
     """A scalar write of M0 and an LDS copy that reads it stand one wait state apart; in inline assembly only the
     source can put it there."""

@@ -229,9 +229,8 @@ class WhisperExt:
 
     def _attn_io_checks(self, q, k, v, out, len_state, k_new, v_new):
         if not _halves(q, k, v, out):
-            if not _halves(q, k, v, out):
-                for t, n in ((q, 'q'), (k, 'k'), (v, 'v'), (out, 'out')):
-                    check_half(t, n)
+            for t, n in ((q, 'q'), (k, 'k'), (v, 'v'), (out, 'out')):
+                check_half(t, n)
         shape = k.shape
         if len(shape) != 3 or shape[2] != HEAD_DIM or v.shape != shape:
             raise RuntimeError('k, v must be [heads, max_len, 64]')

@@ -778,10 +778,11 @@ __global__ void __launch_bounds__(64) attn_combine_kernel(const float* part_m, c
 // decode_attention for caches of up to kDirectKeys keys in one launch: one block per head computes the
 // 64-key splits' wave partials (attn_split_kernel<2>'s: 4 waves of 16 keys a split), merges each split
 // (split_merge) and combines the splits (attn_combine_kernel), all through LDS, so the output is that of
-// the two launches bit for bit. Latency bounds it: 20 blocks of at most 112 KB each. What it saves is the
-// second launch and the partials' trip through memory (448-key cache, 224 keys filled, 20 heads: 4.2 us in
-// the kernel trace against 2.9 + 4.6 us for the two launches). Keys below kDirectFirst are requested before the length is known; the rest, which a
-// cache filled no further does not need, once it is. Longer caches keep the split grid: one CU would
+// the two launches bit for bit, and so is what it leaves in the workspace, if it is given one. Latency bounds
+// it: 20 blocks of at most 112 KB each. What it saves is the second launch and the partials' trip through
+// memory (448-key cache, 224 keys filled, 20 heads: 4.2 us in the kernel trace against 2.9 + 4.6 us for the
+// two launches). Keys below kDirectFirst are requested before the length is known; the rest, which a cache
+// filled no further does not need, once it is. Longer caches keep the split grid: one CU would
 // read a 1500-key head (384 KB) in about 5 us, which takes 24 blocks 1 us.
 // ------------------------------------------------------------------------------------------
 constexpr int kDirectWaves = 16, kDirectKeys = 512;
@@ -840,6 +841,7 @@ __global__ void __launch_bounds__(kDirectWaves * 64) attn_direct_kernel(AttnArgs
       reinterpret_cast<uint4*>(vh + static_cast<size_t>(pos) * kHeadDim)[c] = vnew;
   }
   __syncthreads();
+  const int splits = (a.max_len + kSplitKeys - 1) / kSplitKeys;  // slots per head of the workspace
   if (wave < nsplit) {  // one wave per split (kDirectSplits <= kDirectWaves)
     float m, l, o;
     split_merge<4>(wm + 4 * wave, wl + 4 * wave, wacc + 4 * wave, lane, m, l, o);
@@ -848,6 +850,16 @@ __global__ void __launch_bounds__(kDirectWaves * 64) attn_direct_kernel(AttnArgs
       sm[wave] = m;
       sl[wave] = l;
     }
+    if (a.part_m) {
+      a.part_acc[(head * splits + wave) * kHeadDim + lane] = o;
+      if (lane == 0) {
+        a.part_m[head * splits + wave] = m;
+        a.part_l[head * splits + wave] = l;
+      }
+    }
+  } else if (a.part_m && wave < splits && lane == 0) {  // an empty split
+    a.part_m[head * splits + wave] = -INFINITY;
+    a.part_l[head * splits + wave] = 0.f;
   }
   __syncthreads();
   if (tid >= kHeadDim) return;
@@ -1400,8 +1412,10 @@ extern "C" int fw_decode_attention_noalloc(const void* q, void* k, void* v, void
   rc = noalloc_scratch(&ws);
   if (rc != FW_OK) return rc;
   a.scale = scale;
-  a.part_m = ws;
-  a.part_l = ws + FW_NOALLOC_ATTN_SLOTS;
-  a.part_acc = ws + 2 * FW_NOALLOC_ATTN_SLOTS;
+  if (max_len > kDirectKeys) {  // the one-launch form needs no workspace: calls that overlap do not meet
+    a.part_m = ws;
+    a.part_l = ws + FW_NOALLOC_ATTN_SLOTS;
+    a.part_acc = ws + 2 * FW_NOALLOC_ATTN_SLOTS;
+  }
   return launch_decode_attention(a, nsplit, heads, stream);
 }

@@ -58,8 +58,7 @@ int fw_argmax_finalize(uint64_t* best, int64_t* tokens, int64_t* state, int64_t*
 
 /* Replaces decode_attention (whisper_kernels.cu:300-339, kernels :102-213): split-K single-query
  * attention, 64 keys per split, then a combine launch; caches of up to 512 keys take one launch with the
- * same bits and leave the workspace as it is. q fp16[heads*64]; k, v fp16[heads, max_len, 64];
- * out fp16[heads*64]. Self mode: len_state, k_new, v_new all non-NULL, len = len_state[0] + 1, and the
+ * same bits in out and in the workspace. q fp16[heads*64]; k, v fp16[heads, max_len, 64]; out fp16[heads*64]. Self mode: len_state, k_new, v_new all non-NULL, len = len_state[0] + 1, and the
  * row len_state[0] of k/v is overwritten with k_new/v_new (fp16[heads*64]). Cross mode: all three
  * NULL, len = max_len. part_m/part_l fp32[ws_slots], part_acc fp32[ws_slots*64],
  * ws_slots >= heads * ceil(max_len / 64). */

@@ -222,6 +222,27 @@ def test_decode_attention_one_launch_edges(ext, hip_device, max_len, length, own
     assert np.array_equal(tk.cpu().numpy(), k, equal_nan=True) and np.array_equal(tv.cpu().numpy(), v, equal_nan=True)
 
 
+@pytest.mark.parametrize('max_len,length', [(1, 1), (65, 64), (65, 65), (448, 224), (512, 256), (512, 512), (513, 300)])
+@pytest.mark.parametrize('own', [True, False])
+def test_decode_attention_leaves_the_partials(ext, hip_device, max_len, length, own):
+    """The workspace after decode_attention is that of the split launch alone, bit for bit, in one launch or two:
+    (m, l) of every split, empty ones included, the sums of the splits with keys, and nothing else written."""
+    from flash_whisper_amd.selftest import workspace
+
+    rng = np.random.default_rng(max_len + length)
+    dev, heads = hip_device, 3
+    q, k, v = _attn_inputs(rng, heads, max_len)
+    new = (torch.tensor([length - 1, 0], device=dev), h16(rng.standard_normal((heads, 64)), dev),
+           h16(rng.standard_normal((heads, 64)), dev)) if own else (None, None, None)
+    got, ref = ([t.fill_(7.) for t in workspace(heads, -(-max_len // 64) + 1)] for _ in range(2))
+    out = torch.empty(heads * 64, dtype=torch.float16, device=dev)
+    ext.decode_attention(h16(q, dev), h16(k, dev), h16(v, dev), out, *new, *got, 0.125)
+    ext.attention_split(h16(q, dev), h16(k, dev), h16(v, dev), *new, *ref, 0.125, split_keys=64)
+    assert not bool((ref[0][:heads] == 7).any())
+    for g, r in zip(got, ref):
+        assert torch.equal(g, r)
+
+
 @pytest.mark.parametrize('split_keys,max_len,pos', [(256, 448, 100), (32760, 40000, 32759), (32768, 40000, 32768),
                                                     (65535, 448, 447), (65536, 70000, 65536), (1 << 20, 448, 0),
                                                     (2 ** 31 - 1, 448, 447)])

@@ -983,6 +983,8 @@ int launch_ks(GemmArgs g, int epi, hipStream_t s) {
 //   (1200, 5120, 1280) 128x128 34.3 (2), 192x128 38.0 (2), 256x128 30.4
 //   (251, 1280, 2 x 2560) 64x32 19.4 (2), 64x64 15.1, 96x64 17.7, 128x128 28.4
 //   (400, 1280, 2 x 2560) 64x64 26.1 (2), 96x64 17.6, 128x128 23.1
+// A conv's stage costs what a plain product's does: its sources are per-lane offsets too. The stem's second
+// conv, (769 / 900 / 1000 / 1152, 1280, 3840): 96x64 29.4 / 28.5 / 29.5 / 29.1, 64x128 26.8 / 27.1 / 29.8 / 31.2.
 enum Tile { kD256, kD192, kD128, kD64, kS96x64, kS64x64, kS64x32, kS32x32, kWide256, kTiles };
 struct TileCost {
   int rows, cols;
@@ -1002,9 +1004,7 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
     if (!allowed(static_cast<Tile>(t))) continue;
     const TileCost& c = kTileCost[t];
     const int64_t blocks = static_cast<int64_t>(g.n / c.cols) * ((g.m + c.rows - 1) / c.rows) * (g.splits > 1 ? g.splits : 1);
-    // the direct-to-LDS kernel works out a conv's source rows for every copy
-    const float stage = g.conv_stride && t <= kD64 ? 1.1f * c.per_stage : c.per_stage;
-    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * stage);
+    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * c.per_stage);
     if (best_us == 0.f || us < best_us) {
       best = static_cast<Tile>(t);
       best_us = us;

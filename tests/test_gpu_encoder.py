@@ -178,7 +178,8 @@ def test_gemm_row_strided_views(ext, hip_device):
 
 @pytest.mark.parametrize('stride,c_in,t_in', [(1, 128, 3000), (2, 1280, 3000), (2, 128, 61), (1, 128, 1001), (1, 128, 502),
                                               (1, 64, 1), (2, 1280, 99), (2, 1280, 502), (2, 1280, 1281),
-                                              (1, 128, 1), (2, 1280, 1), (2, 1280, 2)])
+                                              (1, 128, 1), (2, 1280, 1), (2, 1280, 2), (2, 1280, 1601),
+                                              (2, 1280, 2303)])
 def test_conv1d(ext, hip_device, stride, c_in, t_in):
     dev = hip_device
     rng = np.random.default_rng(stride + c_in)

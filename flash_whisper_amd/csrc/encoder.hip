@@ -23,10 +23,10 @@ namespace {
 //  - Plain GEMMs (gemm_dma_kernel): global -> LDS copies into a ring of stages, operand fragments
 //    double-buffered in registers (see the pipeline notes above that kernel).
 //  - Implicit-GEMM conv: a 64-wide k stage of A row m is 64 contiguous channels of input row
-//    m * stride + tap - 1, so convs use the same direct-to-LDS pipeline (padding rows copy from a zero
-//    row).
-//  - Products of few rows: tiles of 32 x 32 to 96 x 64 whose k stages are dealt to the block's waves
-//    (gemm_ks_kernel); choose_tile picks the tile by the passes over the CUs and their cost.
+//    m * stride + tap - 1, so convs use the same direct-to-LDS pipeline, from a raw buffer whose range check
+//    gives the padding rows' zeros (inputs of 2 GiB and more: 64-bit addresses, padding from a zero row).
+//  - Products of few rows: tiles of 32 x 32 to 64 x 64 (split products: 96 x 64) whose k stages are dealt to
+//    the block's waves (gemm_ks_kernel); choose_tile picks the tile by the passes over the CUs and their cost.
 //  - Tile order: hardware deals blocks round-robin over the 8 XCDs; the block id is remapped so each
 //    XCD works on its own part of the tile grid and its L2 sees only that part's operand panels.
 // MFMA 32x32x16 f16 operand layout (lane l, g = l / 32):
@@ -946,8 +946,7 @@ int launch_dma(GemmArgs g, int epi, hipStream_t s) {
 
 template <int TM, int TN, bool CONV>
 int launch_ks(GemmArgs g, int epi, hipStream_t s) {
-  const int tiles = (g.n / TN) * ((g.m + TM - 1) / TM);
-  const dim3 grid(tiles * (g.splits > 1 ? g.splits : 1)), block(kKsWaves * 64);
+  const dim3 grid((g.n / TN) * ((g.m + TM - 1) / TM)), block(kKsWaves * 64);
   choose_xcd_groups(g, TM, TN);
   switch (epi) {
 #define FW_KS_CASE(E, C) \
@@ -962,7 +961,6 @@ int launch_ks(GemmArgs g, int epi, hipStream_t s) {
     FW_KS_CASE(FW_EPI_SCALE_Q, !CONV)
     FW_KS_CASE(kEpiCrossKV, !CONV)
     FW_KS_CASE(kEpiQkvVt, !CONV)
-    FW_KS_CASE(kEpiPartial, !CONV)
 #undef FW_KS_CASE
     default:
       return fw_fail(FW_EINVAL, "gemm: unknown epilogue %d", epi);
@@ -970,10 +968,22 @@ int launch_ks(GemmArgs g, int epi, hipStream_t s) {
   return fw_check_launch(CONV ? "conv1d" : "gemm");
 }
 
+template <int TM, int TN>
+int launch_ks_partial(GemmArgs g, hipStream_t s) {
+  const dim3 grid((g.n / TN) * ((g.m + TM - 1) / TM) * g.splits);
+  choose_xcd_groups(g, TM, TN);
+  hipLaunchKernelGGL((gemm_ks_kernel<TM, TN, kEpiPartial, false>), grid, dim3(kKsWaves * 64), 0, s, FW_GEMM_ARGS(g));
+  return fw_check_launch("gemm_splitk");
+}
+
 // The tile: the fewest passes over the CUs (one block per CU: each tile's ring takes most of its LDS) at
 // the tile's cost, kPassUs + k stages x per_stage. Both are fits to times on MI355X with weights cold (a
 // graph over >300 MB of them; m = 50 .. 1500, n = 1280, 3840, 5120, k = 1280, 2 x 2560 and the convs'
-// 3840), good to about 20%; what decides is mostly the passes. Measured us for (m, n, k) by tile:
+// 3840). The absolute times are rough: over 15 row counts of 7 products the picked tile took 0.67 to 1.25 times
+// what the fit says, the low end where launches are shortest. What decides is mostly the passes: the pick was
+// the fastest or within 2% of it, but for fc2 at 577 and 640 rows (64x64 6% and 9% faster than its 128x128).
+// 96 x 64 serves the split products: of a whole one's 64 x 128 tiles there are never more, and they cost no more.
+// Measured us for (m, n, k) by tile:
 //   (50, 1280, 1280)   32x32 4.8, 64x32 6.2, 64x64 7.8, 64x128 9.6
 //   (251, 1280, 1280)  32x32 7.8 (2 passes), 64x32 6.3, 64x64 8.2, 64x128 10.5, 128x128 15.1
 //   (251, 5120, 1280)  64x64 19.6 (2), 96x64 14.0, 64x128 14.4, 128x128 18.7 (weights in L2: 96x64 11.3, 64x128 9.9)
@@ -1016,11 +1026,10 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
   const bool wide = epi == kEpiCrossKV && g.n % kWide == 0;  // the one epilogue that the wide tiles have
-  switch (choose_tile(g, [&](Tile t) { return t != kWide256 || wide; })) {
+  switch (choose_tile(g, [&](Tile t) { return t != kS96x64 && (t != kWide256 || wide); })) {
     case kD256: return launch_dma<256, kNoConv>(g, epi, s);
     case kD192: return launch_dma<192, kNoConv>(g, epi, s);
     case kD64: return launch_dma<64, kNoConv>(g, epi, s);
-    case kS96x64: return launch_ks<96, 64, false>(g, epi, s);
     case kS64x64: return launch_ks<64, 64, false>(g, epi, s);
     case kS64x32: return launch_ks<64, 32, false>(g, epi, s);
     case kS32x32: return launch_ks<32, 32, false>(g, epi, s);
@@ -1041,13 +1050,10 @@ int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
 // register-staged gather, 10.3 for a 2-deep ring and 10.1 for 128-row tiles; 1000 rows: 6.7, 10.5, 7.8, 9.4).
 int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
   if (!conv_offsets_fit(g) || !copy_offsets_fit(g)) return launch_dma<128, kConvAny>(g, epi, s);
-  switch (choose_tile(g, [&](Tile t) { return t >= kD128 && t != kWide256; })) {
+  switch (choose_tile(g, [&](Tile t) { return t >= kD128 && t != kS96x64 && t != kWide256; })) {
     case kS64x64: return launch_ks<64, 64, true>(g, epi, s);
     case kS64x32: return launch_ks<64, 32, true>(g, epi, s);
     case kS32x32: return launch_ks<32, 32, true>(g, epi, s);
-    case kS96x64:
-      if (g.k >= 1024) return launch_ks<96, 64, true>(g, epi, s);
-      break;
     case kD64:
       if (g.k >= 1024) return launch_dma<64, kConvBuffer>(g, epi, s);
       break;
@@ -1275,10 +1281,10 @@ extern "C" int fw_gemm_splitk(const void* a, int lda, const void* w, int ldw, fl
   g.part = part;
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm_splitk: each operand must span less than 4 GiB");
   switch (choose_tile(g, [](Tile t) { return t == kD128 || (t > kD64 && t != kWide256); })) {
-    case kS96x64: return launch_ks<96, 64, false>(g, kEpiPartial, stream);
-    case kS64x64: return launch_ks<64, 64, false>(g, kEpiPartial, stream);
-    case kS64x32: return launch_ks<64, 32, false>(g, kEpiPartial, stream);
-    case kS32x32: return launch_ks<32, 32, false>(g, kEpiPartial, stream);
+    case kS96x64: return launch_ks_partial<96, 64>(g, stream);
+    case kS64x64: return launch_ks_partial<64, 64>(g, stream);
+    case kS64x32: return launch_ks_partial<64, 32>(g, stream);
+    case kS32x32: return launch_ks_partial<32, 32>(g, stream);
     default: break;
   }
   // the XCD rectangles of the plain GEMMs (both k halves of a tile land on the same XCD when the tile

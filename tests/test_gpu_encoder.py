@@ -65,17 +65,19 @@ def test_gemm_epilogues(ext, hip_device, m, n, k, epi):
     close_rel(np32(out), ref, scale=scale)
 
 
-# few rows: the sliced tiles (32 x 32, 64 x 32, 64 x 64 and 96 x 64 in turn), fewer k stages than waves, a
-# count of stages that does not divide by the waves, and partial last row tiles
+# few rows: the sliced tiles (32 x 32 up to 97 rows, 64 x 32 for (251, 1280), 64 x 64 for (129, 3840)) and the
+# 64 x 128 ones past them (251, 5120); fewer k stages than waves, a count of stages that does not divide by the
+# waves, and partial last row tiles
 @pytest.mark.parametrize('m,n,k,epi', [(1, 128, 64, 0), (33, 1280, 64, 4), (50, 1280, 1280, 2), (97, 1280, 192, 3),
                                        (251, 1280, 1280, 2), (129, 3840, 1280, 5), (251, 5120, 1280, 1)])
 def test_gemm_few_rows(ext, hip_device, m, n, k, epi):
     test_gemm_epilogues(ext, hip_device, m, n, k, epi)
 
 
-@pytest.mark.parametrize('m', [1, 64, 65, 251, 400, 577])
+@pytest.mark.parametrize('m', [1, 64, 65, 100, 251, 400, 577])
 def test_gemm_splitk_few_rows(ext, hip_device, m):
-    """Both k halves of fc2 by the sliced tiles (and 128-row tiles at 577), each against its own product."""
+    """Both k halves of fc2 by the sliced tiles (32 x 32 up to 65 rows, then 64 x 32, 64 x 64, 96 x 64; 128-row
+    tiles at 577), each against its own product."""
     dev = hip_device
     rng = np.random.default_rng(m)
     a, w = np.float16(0.5 * rng.standard_normal((m, 5120))), np.float16(0.02 * rng.standard_normal((1280, 5120)))
@@ -179,7 +181,7 @@ def test_gemm_row_strided_views(ext, hip_device):
 @pytest.mark.parametrize('stride,c_in,t_in', [(1, 128, 3000), (2, 1280, 3000), (2, 128, 61), (1, 128, 1001), (1, 128, 502),
                                               (1, 64, 1), (2, 1280, 99), (2, 1280, 502), (2, 1280, 1281),
                                               (1, 128, 1), (2, 1280, 1), (2, 1280, 2), (2, 1280, 1601),
-                                              (2, 1280, 2303)])
+                                              (2, 1280, 2303), (2, 1280, 3301)])
 def test_conv1d(ext, hip_device, stride, c_in, t_in):
     dev = hip_device
     rng = np.random.default_rng(stride + c_in)
@@ -198,6 +200,27 @@ def test_conv1d(ext, hip_device, stride, c_in, t_in):
         scale = np.abs(ref) + np.abs(pos.astype(np.float32))
         ref = f16(ref + pos.astype(np.float32))
     close_rel(np32(out), ref, scale=scale)
+
+
+@pytest.mark.parametrize('stride,t_in', [(1, 838859), (1, 838860), (2, 838861)])
+def test_conv1d_of_two_gib(ext, hip_device, stride, t_in):
+    """Either side of where input and padding row reach 2 GiB (838860 rows of 1280 channels) and 64-bit addresses
+    take over from the raw buffer: the rows at the input's ends and its middle against their product in 64 bits."""
+    c_in, c_out = 1280, 128
+    x = torch.empty(t_in, c_in, dtype=torch.float16, device=hip_device)
+    x.normal_(generator=torch.Generator(device=hip_device).manual_seed(stride))
+    rng = np.random.default_rng(stride)
+    wp, b = h16(0.02 * rng.standard_normal((c_out, 3 * c_in)), hip_device), h16(rng.standard_normal(c_out), hip_device)
+    t_out = (t_in - 1) // stride + 1
+    out = torch.empty(t_out, c_out, dtype=torch.float16, device=hip_device)
+    ext.conv1d(x, stride, wp, b, out, 0)
+    rows = [0, 1, 2, 127, 128, t_out // 2, t_out // 2 + 1, t_out - 129, t_out - 3, t_out - 2, t_out - 1]
+    zero = torch.zeros(c_in, dtype=torch.float16, device=hip_device)
+    taps = torch.stack([torch.cat([x[r] if 0 <= r < t_in else zero for r in range(m * stride - 1, m * stride + 2)])
+                        for m in rows])
+    ref = taps.double() @ wp.double().T + b.double()
+    close_rel(np32(out[rows]), ref.cpu().numpy())
+    assert bool(torch.isfinite(out).all())
 
 
 def test_layernorm_rows(ext, hip_device):
@@ -263,10 +286,12 @@ def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m):
     assert torch.equal(vt, vt_ref)
 
 
-@pytest.mark.parametrize('t,layers', [(1500, 4), (1025, 3), (1281, 4)])
-def test_cross_kv_wide_tiles_match_gemm(ext, hip_device, t, layers):
-    """Sizes that take the 256 x 256 tiles (whole and partial last row tiles): the bits of the plain product,
-    whose tiles add the same terms in the same order, in the cache layout."""
+# 256 x 256 tiles first, whole and partial last row tiles, then each of the others: 32 x 32, 64 x 32, 64 x 64,
+# 64 x 128, 128 x 128, 192 x 128, 256 x 128
+@pytest.mark.parametrize('t,layers', [(1500, 4), (1025, 3), (1281, 4), (50, 1), (100, 1), (251, 1), (100, 4), (251, 4),
+                                      (400, 4), (577, 4)])
+def test_cross_kv_matches_gemm(ext, hip_device, t, layers):
+    """The bits of the plain product, whose tiles add the same terms in the same order, in the cache layout."""
     rng = np.random.default_rng(t)
     enc = h16(rng.standard_normal((t, 1280)), hip_device)
     n = layers * 2 * 1280

@@ -884,9 +884,16 @@ __global__ void __launch_bounds__(kDirectWaves * 64) attn_direct_kernel(AttnArgs
   a.out[head * kHeadDim + tid] = f2h(num / den);
 }
 
-// The 64-key splits and their combine: one launch while a head's keys fit one block's two rounds.
+// The 64-key splits and their combine: one launch while a head's keys fit one block's two rounds, but for a
+// single split of so many heads that its block of 16 waves, 12 of them without keys, is what costs (us in one
+// launch / two, 64 keys: 512 heads 5.0 / 6.5, 1024 heads 8.4 / 8.1, 2048 heads 14.2 / 11.1; 128 keys: 1024 heads
+// 10.6 / 11.2, 2048 heads 15.0 / 15.2).
+bool attention_in_one_launch(int max_len, int heads) {
+  return max_len <= kDirectKeys && (max_len > kSplitKeys || heads < 1024);
+}
+
 int launch_decode_attention(const AttnArgs& a, int nsplit, int heads, hipStream_t s) {
-  if (a.max_len <= kDirectKeys) {
+  if (attention_in_one_launch(a.max_len, heads)) {
     hipLaunchKernelGGL(attn_direct_kernel, dim3(heads), dim3(kDirectWaves * 64), 0, s, a);
     return fw_check_launch("decode_attention");
   }
@@ -1412,7 +1419,7 @@ extern "C" int fw_decode_attention_noalloc(const void* q, void* k, void* v, void
   rc = noalloc_scratch(&ws);
   if (rc != FW_OK) return rc;
   a.scale = scale;
-  if (max_len > kDirectKeys) {  // the one-launch form needs no workspace: calls that overlap do not meet
+  if (!attention_in_one_launch(max_len, heads)) {  // else no workspace: calls that overlap do not meet
     a.part_m = ws;
     a.part_l = ws + FW_NOALLOC_ATTN_SLOTS;
     a.part_acc = ws + 2 * FW_NOALLOC_ATTN_SLOTS;

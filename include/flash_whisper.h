@@ -57,10 +57,12 @@ int fw_argmax_finalize(uint64_t* best, int64_t* tokens, int64_t* state, int64_t*
                        hipStream_t stream);
 
 /* Replaces decode_attention (whisper_kernels.cu:300-339, kernels :102-213): split-K single-query
- * attention, 64 keys per split, then a combine launch; caches of up to 512 keys take one launch with the
- * same bits in out and in the workspace. q fp16[heads*64]; k, v fp16[heads, max_len, 64]; out fp16[heads*64]. Self mode: len_state, k_new, v_new all non-NULL, len = len_state[0] + 1, and the
- * row len_state[0] of k/v is overwritten with k_new/v_new (fp16[heads*64]). Cross mode: all three
- * NULL, len = max_len. part_m/part_l fp32[ws_slots], part_acc fp32[ws_slots*64],
+ * attention, 64 keys per split, then a combine launch; caches of up to 512 keys take one launch (but for
+ * 1024 heads and more of at most 64 keys) with the same bits in out and in the workspace. q fp16[heads*64];
+ * k, v fp16[heads, max_len, 64]; out fp16[heads*64]. Self mode: len_state, k_new, v_new all non-NULL,
+ * len = len_state[0] + 1, and the row len_state[0] of k/v is overwritten with k_new/v_new
+ * (fp16[heads*64]). Cross mode: all three NULL, len = max_len. part_m/part_l fp32[ws_slots],
+ * part_acc fp32[ws_slots*64],
  * ws_slots >= heads * ceil(max_len / 64). */
 int fw_decode_attention(const void* q, void* k, void* v, void* out, const int64_t* len_state,
                         const void* k_new, const void* v_new, int heads, int max_len, float* part_m,
@@ -68,9 +70,9 @@ int fw_decode_attention(const void* q, void* k, void* v, void* out, const int64_
 
 /* fw_decode_attention without the workspace arguments, for callers that cannot allocate (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc); it has no counterpart in
- * the reference. Same kernels and the same result, bit for bit. Past 512 keys the split partials live
- * in a static device array of this library: FW_NOALLOC_ATTN_SLOTS (head, split) slots, 528 KiB on each
- * GPU the library runs on, held until the process ends. heads * ceil(max_len / 64) above
+ * the reference. Same kernels and the same result, bit for bit. Where two launches run, the split partials
+ * live in a static device array of this library: FW_NOALLOC_ATTN_SLOTS (head, split) slots, 528 KiB on
+ * each GPU the library runs on, held until the process ends. heads * ceil(max_len / 64) above
  * FW_NOALLOC_ATTN_SLOTS fails with FW_EINVAL before any launch. The array's address on a device is
  * looked up at the first call on that device; no call allocates or frees memory. Calls on one GPU share
  * the array: calls that overlap on one GPU (different streams) race. */

@@ -243,6 +243,26 @@ def test_decode_attention_leaves_the_partials(ext, hip_device, max_len, length, 
         assert torch.equal(g, r)
 
 
+@pytest.mark.parametrize('max_len', [64, 65])
+def test_decode_attention_of_many_heads(ext, hip_device, max_len):
+    """1024 heads of one split take two launches, of two splits (and 512 heads) one: the same bits, with a
+    workspace and without."""
+    from flash_whisper_amd.selftest import workspace
+
+    rng = np.random.default_rng(max_len)
+    dev, heads = hip_device, 1024
+    q, k, v = (h16(t, dev) for t in _attn_inputs(rng, heads, max_len))
+    state, new = torch.tensor([40, 0], device=dev), h16(rng.standard_normal((heads, 64)), dev)
+    ref = torch.empty(heads * 64, dtype=torch.float16, device=dev)
+    for c in (slice(0, 512), slice(512, 1024)):
+        e = slice(64 * c.start, 64 * c.stop)
+        ext.decode_attention(q[e], k[c].clone(), v[c].clone(), ref[e], state, new[c], new[c], *workspace(512, 2), 0.125)
+    out, out2 = torch.empty_like(ref), torch.empty_like(ref)
+    ext.decode_attention(q, k.clone(), v.clone(), out, state, new, new, *workspace(heads, 2), 0.125)
+    ext.decode_attention_noalloc(q, k.clone(), v.clone(), out2, state, new, new, 0.125)
+    assert torch.equal(out, ref) and torch.equal(out2, ref)
+
+
 @pytest.mark.parametrize('split_keys,max_len,pos', [(256, 448, 100), (32760, 40000, 32759), (32768, 40000, 32768),
                                                     (65535, 448, 447), (65536, 70000, 65536), (1 << 20, 448, 0),
                                                     (2 ** 31 - 1, 448, 447)])

@@ -226,11 +226,17 @@ void launch_gemv_batch(int nv, const _Float16* x, const LnArgs& ln, const Combin
 #ifndef FW_GK5120_NW
 #define FW_GK5120_NW 5  // fc2 (K = 5120): 5 rows per block
 #endif
+#ifndef FW_GK5120_WIDE_NW
+#define FW_GK5120_WIDE_NW 8  // past gk5120_narrow's rows
+#endif
 #ifndef FW_GK5120_U
 #define FW_GK5120_U 1
 #endif
 #ifndef FW_CMB_NW
 #define FW_CMB_NW 8  // combine + out projection: 16 rows per block
+#endif
+#ifndef FW_CMB_WIDE_NW
+#define FW_CMB_WIDE_NW 12  // batches, and past cmb_narrow's rows: 24 rows per block
 #endif
 // Block shapes are whole blocks within the 1024-thread launch bound with at least one row group per
 // wave; any such shape computes the same rows (each row's lane split and order depend on K only).
@@ -239,9 +245,17 @@ void launch_gemv_batch(int nv, const _Float16* x, const LnArgs& ln, const Combin
 #define FW_GEMV_SHAPE_OK(NW, U) ((NW) >= 1 && (NW) <= 16 && (U) >= 1 && (U) <= 4)
 static_assert(FW_GEMV_SHAPE_OK(FW_G5120_NW, FW_G5120_U) && FW_GEMV_SHAPE_OK(FW_G3840_NW, FW_G3840_U) &&
                   FW_GEMV_SHAPE_OK(FW_G1280_NW, 1) && FW_GEMV_SHAPE_OK(FW_GK5120_NW, FW_GK5120_U) &&
-                  FW_GEMV_SHAPE_OK(FW_CMB_NW, 1),
+                  FW_GEMV_SHAPE_OK(FW_GK5120_WIDE_NW, 1) && FW_GEMV_SHAPE_OK(FW_CMB_NW, 1) &&
+                  FW_GEMV_SHAPE_OK(FW_CMB_WIDE_NW, 1),
               "decode GEMV block shapes: 1..16 waves, 1..4 row groups per wave");
 #undef FW_GEMV_SHAPE_OK
+// Where the two shapes of K = 5120 and of the combine cross over (weights from HBM, us a launch in a graph).
+// fc2, 5 waves / 8, one vector: 1280 rows 4.1 / 4.6, 2560 6.2 / 7.6, 5120 9.3 / 9.8, 20000 35.2 / 34.7; four
+// vectors: 2560 9.5 / 11.0, 3840 12.6 / 11.8, 20000 58 / 51: each block reads its input vectors anew, so with
+// many of both more rows should share them. The combine is per block: one vector, 8 waves / 12, 7 splits: 1280
+// rows 3.4 / 3.7, 3840 4.0 / 4.2, 5120 5.2 / 4.9; four vectors: 1280 8.7 / 8.4, 5120 16.5 / 9.7.
+bool gk5120_narrow(int n, int nv) { return n <= (nv == 1 ? 5120 : 2560); }
+bool cmb_narrow(int n, int nv) { return nv == 1 && n <= 3840; }
 template <int MODE, int ACT>
 void dispatch_gemv_1280(const _Float16* x, const LnArgs& ln, const CombineArgs& cb, const _Float16* w,
                         const _Float16* b, _Float16* out, int n, hipStream_t s) {
@@ -264,6 +278,20 @@ void dispatch_gemv_1280_batch(int nv, const _Float16* x, const LnArgs& ln, const
     launch_gemv_batch<kHidden, FW_G3840_NW, MODE, ACT>(nv, x, ln, cb, w, b, out, n, s);
   else
     launch_gemv_batch<kHidden, FW_G1280_NW, MODE, ACT>(nv, x, ln, cb, w, b, out, n, s);
+}
+
+template <int ACT>
+void launch_gemv_5120(int nv, const _Float16* x, const _Float16* w, const _Float16* b, _Float16* out, int n,
+                      hipStream_t s) {
+  constexpr int K = 4 * kHidden;
+  const LnArgs ln{};
+  const CombineArgs cb{};
+  if (!gk5120_narrow(n, nv))
+    launch_gemv_batch<K, FW_GK5120_WIDE_NW, kModePlain, ACT>(nv, x, ln, cb, w, b, out, n, s);
+  else if (nv == 1)
+    launch_gemv<K, FW_GK5120_NW, FW_GK5120_U, kModePlain, ACT>(x, ln, cb, w, b, out, n, s);
+  else
+    launch_gemv_batch<K, FW_GK5120_NW, kModePlain, ACT>(nv, x, ln, cb, w, b, out, n, s);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1207,16 +1235,10 @@ static int gemv_impl(const void* x, const void* w, const void* bias, void* out, 
       dispatch_gemv_1280_batch<kModePlain, FW_ACT_GELU>(nv, xp, ln, cb, wp, bp, op, n_out, stream);
     else
       dispatch_gemv_1280_batch<kModePlain, FW_ACT_NONE>(nv, xp, ln, cb, wp, bp, op, n_out, stream);
-  } else if (nv == 1) {
-    if (act == FW_ACT_GELU)
-      launch_gemv<4 * kHidden, FW_GK5120_NW, FW_GK5120_U, kModePlain, FW_ACT_GELU>(xp, ln, cb, wp, bp, op, n_out, stream);
-    else
-      launch_gemv<4 * kHidden, FW_GK5120_NW, FW_GK5120_U, kModePlain, FW_ACT_NONE>(xp, ln, cb, wp, bp, op, n_out, stream);
+  } else if (act == FW_ACT_GELU) {
+    launch_gemv_5120<FW_ACT_GELU>(nv, xp, wp, bp, op, n_out, stream);
   } else {
-    if (act == FW_ACT_GELU)
-      launch_gemv_batch<4 * kHidden, FW_GK5120_NW, kModePlain, FW_ACT_GELU>(nv, xp, ln, cb, wp, bp, op, n_out, stream);
-    else
-      launch_gemv_batch<4 * kHidden, FW_GK5120_NW, kModePlain, FW_ACT_NONE>(nv, xp, ln, cb, wp, bp, op, n_out, stream);
+    launch_gemv_5120<FW_ACT_NONE>(nv, xp, wp, bp, op, n_out, stream);
   }
   return fw_check_launch("gemv");
 }
@@ -1339,11 +1361,11 @@ static int attn_out_gemv_impl(const float* part_m, const float* part_l, const fl
   const auto* wp = static_cast<const _Float16*>(w);
   const auto* bp = static_cast<const _Float16*>(bias);
   auto* op = static_cast<_Float16*>(out);
-  if (nv == 1)
+  if (cmb_narrow(n_out, nv))
     launch_gemv<kHidden, FW_CMB_NW, 1, kModeCombine, FW_ACT_NONE>(nullptr, LnArgs{}, cb, wp, bp, op, n_out, stream);
   else
-    launch_gemv_batch<kHidden, FW_CMB_NW, kModeCombine, FW_ACT_NONE>(nv, nullptr, LnArgs{}, cb, wp, bp, op, n_out,
-                                                                     stream);
+    launch_gemv_batch<kHidden, FW_CMB_WIDE_NW, kModeCombine, FW_ACT_NONE>(nv, nullptr, LnArgs{}, cb, wp, bp, op, n_out,
+                                                                          stream);
   return fw_check_launch("attn_out_gemv");
 }
 

@@ -111,6 +111,34 @@ def test_gemv_block_edges(ext, hip_device, n):
         assert torch.equal(out[:n], full[:n]) and bool((out[n:] == 7).all())
 
 
+@pytest.mark.parametrize('n', [2560, 2561, 3840, 3841, 5120, 5121])
+@pytest.mark.parametrize('nv', [1, 2, 4])
+def test_gemv_block_shapes(ext, hip_device, n, nv):
+    """Row counts either side of where the blocks of fc2 and of the combine + out projection change shape, single
+    and batched: each vector's first 128 rows as a call for those rows gives them, bit for bit."""
+    dev, heads = hip_device, 20
+    g = torch.Generator(device=dev).manual_seed(n + nv)
+    m, l, acc = (torch.rand(nv * heads * k, generator=g, device=dev) + 0.5 for k in (7, 7, 7 * 64))
+    x = torch.randn(nv, 5120, generator=g, device=dev).half()
+
+    def fc2(w, b, out):
+        ext.gemv(x.view(-1) if nv == 1 else x, w, b, out, nv=nv)
+
+    def attn_out(w, b, out):
+        ext.attn_out_gemv(m, l, acc, None, heads, 448, w, b, out, split_keys=64, nv=nv)
+
+    for op, k in ((fc2, 5120), (attn_out, 1280)):
+        w = torch.randn(n, k, generator=g, device=dev).mul_(0.02).half()
+        b = torch.randn(n, generator=g, device=dev).half()
+        out, part = (torch.full((nv, r), 7., dtype=torch.float16, device=dev) for r in (n, 128))
+        op(w, b, out)
+        op(w[:128], b[:128], part)
+        assert torch.equal(out[:, :128], part)
+        ref = (x.double() if op is fc2 else (acc.view(nv, heads, 7, 64) * (m.exp().view(nv, heads, 7, 1))).sum(2).div(
+            (l * m.exp()).view(nv, heads, 7).sum(2, keepdim=True)).view(nv, 1280).half().double()) @ w.double().T + b
+        close_rel(np32(out), ref.cpu().numpy())
+
+
 @pytest.mark.parametrize('n,act,embed', [(3840, 0, False), (1280, 0, False), (5120, 1, False), (3840, 0, True)])
 def test_ln_gemv(ext, hip_device, n, act, embed):
     from oracle.common import f16, gelu

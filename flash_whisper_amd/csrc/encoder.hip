@@ -832,8 +832,13 @@ __global__ void __launch_bounds__(kKsWaves * 64) gemm_ks_kernel(FW_GEMM_PARAMS) 
   if constexpr (EPI == kEpiQkvVt) {
     if (n0 >= 2 * g.q_cols) {  // a tile of v columns: 4 adjacent keys of one column per thread, stored transposed
       _Float16* dst = g.vt + static_cast<size_t>(n0 - 2 * g.q_cols) * g.vt_pad;
+      // a wave takes 16 keys of 16 columns at a time: its reads of the sums meet in no LDS bank (4 rows are 16
+      // banks on), and 4 lanes store 32 bytes of a column (a column's 64 keys a quarter-wave: every read 4-way)
+      static_assert(4 * kRowF % 64 == 16, "4 rows of sums are 16 banks on");
+#pragma unroll
       for (int c = tid; c < TM / 4 * TN; c += kKsWaves * 64) {
-        const int col = c / (TM / 4), rl = c % (TM / 4) * 4;  // rows rl .. rl + 3 stay adjacent under vt_pos
+        const int blk = c >> 6, col = blk / (TM / 16) * 16 + (c >> 2 & 15);
+        const int rl = blk % (TM / 16) * 16 + (c & 3) * 4;  // rows rl .. rl + 3 stay adjacent under vt_pos
         const float b = g.bias ? h2f(g.bias[n0 + col]) : 0.f;
         h4v o;
 #pragma unroll

@@ -1011,16 +1011,28 @@ constexpr TileCost kTileCost[kTiles] = {{256, 128, 1.15f}, {192, 128, 0.85f}, {1
 constexpr float kPassUs = 4.f;
 constexpr int kCus = 256;
 
+// What the fit leaves out, us by both tiles:
+//  - 64 x 64 and 96 x 64 sliced tiles with fewer k stages than waves: the idle waves' sums are added all the same
+//    ((400, 1280, 64) 64x64 4.9, 64x128 4.5; (6000, 128, 2 x 64) 96x64 5.3, 128x128 4.5; four stages even).
+//  - q/k/v on 64 x 64 sliced tiles: kVtUs a pass for V^T, stored 8 bytes a lane ((500, 1152, 384) 5.6, 64x128 5.2;
+//    (333, 1536, 512) 6.1, 6.1; (251, 3840, 1280) 10.6, 13.4). Its unfused form too, so that both give the same bits.
+//  - Three passes or more of 256-row tiles cost less than that many single ones: they stay up to kManyPasses of
+//    the best ((8000, 3840, 1280) 113, 192x128 120; (8000, 2560, 5120) 239, 192x128 254, 128x128 256).
+constexpr float kVtUs = 1.5f, kManyPasses = 1.08f;
+
 template <class Allowed>
-Tile choose_tile(const GemmArgs& g, Allowed allowed) {
+Tile choose_tile(const GemmArgs& g, Allowed allowed, bool vt = false) {
   Tile best = kD128;
   float best_us = 0.f;
-  for (int t = 0; t < kTiles; ++t) {
-    if (!allowed(static_cast<Tile>(t))) continue;
+  const bool few_stages = g.k < kKsWaves * kBK;
+  for (int t = kTiles - 1; t >= 0; --t) {  // the 256-row tile last
+    if (!allowed(static_cast<Tile>(t)) || (few_stages && (t == kS64x64 || t == kS96x64))) continue;
     const TileCost& c = kTileCost[t];
     const int64_t blocks = static_cast<int64_t>(g.n / c.cols) * ((g.m + c.rows - 1) / c.rows) * (g.splits > 1 ? g.splits : 1);
-    const float us = static_cast<float>((blocks + kCus - 1) / kCus) * (kPassUs + static_cast<float>(g.k / kBK) * c.per_stage);
-    if (best_us == 0.f || us < best_us) {
+    const int64_t passes = (blocks + kCus - 1) / kCus;
+    const float pass_us = kPassUs + static_cast<float>(g.k / kBK) * c.per_stage + (vt && t == kS64x64 ? kVtUs : 0.f);
+    const float us = static_cast<float>(passes) * pass_us;
+    if (best_us == 0.f || us <= best_us || (t == kD256 && passes >= 3 && us < kManyPasses * best_us)) {
       best = static_cast<Tile>(t);
       best_us = us;
     }
@@ -1031,7 +1043,8 @@ Tile choose_tile(const GemmArgs& g, Allowed allowed) {
 int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
   if (!copy_offsets_fit(g)) return fw_fail(FW_EINVAL, "gemm: each operand must span less than 4 GiB");
   const bool wide = epi == kEpiCrossKV && g.n % kWide == 0;  // the one epilogue that the wide tiles have
-  switch (choose_tile(g, [&](Tile t) { return t != kS96x64 && (t != kWide256 || wide); })) {
+  switch (choose_tile(g, [&](Tile t) { return t != kS96x64 && (t != kWide256 || wide); },
+                      epi == kEpiQkvVt || epi == FW_EPI_SCALE_Q)) {
     case kD256: return launch_dma<256, kNoConv>(g, epi, s);
     case kD192: return launch_dma<192, kNoConv>(g, epi, s);
     case kD64: return launch_dma<64, kNoConv>(g, epi, s);

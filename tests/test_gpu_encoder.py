@@ -69,9 +69,23 @@ def test_gemm_epilogues(ext, hip_device, m, n, k, epi):
 # 64 x 128 ones past them (251, 5120); fewer k stages than waves, a count of stages that does not divide by the
 # waves, and partial last row tiles
 @pytest.mark.parametrize('m,n,k,epi', [(1, 128, 64, 0), (33, 1280, 64, 4), (50, 1280, 1280, 2), (97, 1280, 192, 3),
-                                       (251, 1280, 1280, 2), (129, 3840, 1280, 5), (251, 5120, 1280, 1)])
+                                       (251, 1280, 1280, 2), (129, 3840, 1280, 5), (251, 5120, 1280, 1),
+                                       (400, 1280, 192, 1), (400, 1280, 256, 1)])
 def test_gemm_few_rows(ext, hip_device, m, n, k, epi):
     test_gemm_epilogues(ext, hip_device, m, n, k, epi)
+
+
+@pytest.mark.parametrize('m,n,k', [(150, 128, 128), (400, 1280, 128), (400, 1280, 512), (6000, 128, 128)])
+def test_gemm_splitk_few_stages(ext, hip_device, m, n, k):
+    """Splits of one k stage and of as many as a sliced tile has waves, either side of where the larger sliced
+    tiles are left out."""
+    rng = np.random.default_rng(m)
+    a, w = np.float16(0.5 * rng.standard_normal((m, k))), np.float16(0.02 * rng.standard_normal((n, k)))
+    part = torch.full((2, m, n), float('nan'), dtype=torch.float32, device=hip_device)
+    ext.gemm_splitk(h16(a, hip_device), h16(w, hip_device), part)
+    for half in range(2):
+        c = slice(k // 2 * half, k // 2 * (half + 1))
+        close_rel(np32(part[half]), a[:, c].astype(np.float64) @ w[:, c].astype(np.float64).T, rtol=1e-4)
 
 
 @pytest.mark.parametrize('m', [1, 64, 65, 100, 251, 400, 577])
@@ -265,24 +279,26 @@ def test_encoder_attention(ext, hip_device, seq, heads, qscale):
     close_rel(np32(out), _attn_ref(qkv, heads))
 
 
-@pytest.mark.parametrize('m', [1500, 77, 1, 65, 97, 130, 251])
-def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m):
+@pytest.mark.parametrize('m,heads', [(1500, 20), (77, 20), (1, 20), (65, 20), (97, 20), (130, 20), (251, 20),
+                                     (1500, 2), (800, 4), (500, 6), (333, 8), (333, 10), (251, 12)])
+def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m, heads):
     """The fused q/k/v projection writes the FW_EPI_SCALE_Q GEMM's q and k columns and, for v, exactly
-    what fw_encoder_pack_vt makes of that GEMM's v columns (padding keys zero)."""
-    dev = hip_device
+    what fw_encoder_pack_vt makes of that GEMM's v columns (padding keys zero); with fewer heads on either side
+    of where 64 x 64 tiles give way to 64 x 128."""
+    dev, d = hip_device, 64 * heads
     rng = np.random.default_rng(m)
-    y = h16(np.float16(rng.standard_normal((m, 1280))), dev)
-    w = h16(np.float16(0.02 * rng.standard_normal((3840, 1280))), dev)
-    b = h16(np.float16(0.02 * rng.standard_normal(3840)), dev)
-    ref = torch.empty(m, 3840, dtype=torch.float16, device=dev)
-    ext.gemm(y, w, b, ref, 5, q_cols=1280)
-    vt_ref = ext.encoder_vt_workspace(m, 20)
-    ext.encoder_pack_vt(ref, vt_ref, 20)
-    qkv = torch.full((m, 3840), 7.0, dtype=torch.float16, device=dev)
+    y = h16(np.float16(rng.standard_normal((m, d))), dev)
+    w = h16(np.float16(0.02 * rng.standard_normal((3 * d, d))), dev)
+    b = h16(np.float16(0.02 * rng.standard_normal(3 * d)), dev)
+    ref = torch.empty(m, 3 * d, dtype=torch.float16, device=dev)
+    ext.gemm(y, w, b, ref, 5, q_cols=d)
+    vt_ref = ext.encoder_vt_workspace(m, heads)
+    ext.encoder_pack_vt(ref, vt_ref, heads)
+    qkv = torch.full((m, 3 * d), 7.0, dtype=torch.float16, device=dev)
     vt = torch.full_like(vt_ref, float('nan'))
-    ext.encoder_qkv(y, w, b, qkv, vt, 20)
-    assert torch.equal(qkv[:, :2560], ref[:, :2560])
-    assert torch.equal(qkv[:, 2560:], torch.full_like(qkv[:, 2560:], 7.0))  # v columns untouched
+    ext.encoder_qkv(y, w, b, qkv, vt, heads)
+    assert torch.equal(qkv[:, :2 * d], ref[:, :2 * d])
+    assert torch.equal(qkv[:, 2 * d:], torch.full_like(qkv[:, 2 * d:], 7.0))  # v columns untouched
     assert torch.equal(vt, vt_ref)
 
 

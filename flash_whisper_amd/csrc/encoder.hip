@@ -533,6 +533,7 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(FW_GEMM
   // Against storing from the registers (2 bytes of a column each, 8 bytes on 64-row tiles): a product with
   // a single k stage 4.3 -> 3.8 us at 1500 x 1280, 6.1 -> 5.8 us at 1500 x 3840, 7.45 us as before at
   // 1500 x 5120, where writing 15 MB takes that long either way; the encoder 4034 -> 4012 us.
+  // Where it costs: GELU products of short k over many rows (3000 x 5120, k = 320: 28.9 -> 30.1 us).
   if constexpr (EPI == kEpiPartial) {
     constexpr int kRowF = kBN + 4;
     static_assert(BM * kRowF * 4 <= kDmaStages * kStageBytes, "staging tile must fit the ring");
@@ -598,8 +599,8 @@ __global__ void __launch_bounds__(gemm_waves<BM>() * 64) gemm_dma_kernel(FW_GEMM
 // The cross K/V of 3 or 4 decoder layers: products so wide that 256 x 128 tiles take two passes over the
 // CUs. 2 x 4 waves of 128 x 64, a ring of two 64 KB stages; a stage's operands are read 16 of k at a time,
 // double-buffered in registers, and the last 16 are multiplied behind the barrier of the next stage, while
-// its first are read. A tile moves 2/3 of the bytes per product of a 256 x 128 one, which matters where
-// power sets the clock (about 1.9 GHz in these products). 1500 x 10240 x 1280: 47.8 -> 41.1 us a call.
+// its first are read. A tile moves 2/3 of the bytes per product of a 256 x 128 one and makes 3/4 of
+// the LDS reads: MFMAs busy 37% against 31.5%. 1500 x 10240 x 1280: 47.8 -> 41.1 us a call.
 constexpr int kWideWaves = 8, kWide = 256, kWideStage = 2 * kWide * 128;
 constexpr int kWideRowH = kWide + 8;  // halves per staged output row
 constexpr int kWideLds = kWide * kWideRowH * 2 > 2 * kWideStage ? kWide * kWideRowH * 2 : 2 * kWideStage;
@@ -1085,8 +1086,10 @@ int launch_conv(const GemmArgs& g, int epi, hipStream_t s) {
 // Row LayerNorm over 1280 columns: 32 lanes per row (5 x 16-byte chunks each), kLnRows = kLnThreads / 32 rows per block.
 // ------------------------------------------------------------------------------------------
 constexpr int kLnC = kHidden / 8 / 32;  // 16-byte fp16 chunks per lane of a row
-// One wave (two rows) a block: 251 rows make 126 blocks instead of 32 (the encoder over 251 frames 295.6 ->
-// 291.2 us, over 1500 frames 4292 -> 4284 us; 128 threads 292.1 and 4315 us).
+// One wave (two rows) a block for both kernels: 251 rows make 126 blocks instead of 32. Four encoder layers over
+// 251 frames take 245.3 us, with 256 threads in both 249.9, in the plain one alone 246.9, in the residual one
+// alone 249.1; over 50 frames 157.5 and 161.0; over 500 to 1500 frames all within 0.5%. Chains of either alone
+// are the fastest at 64 threads from 1 to 20000 rows (1500 rows: plain 3.5 against 3.7 us, residual 5.1, 5.6).
 #ifndef FW_LN_THREADS
 #define FW_LN_THREADS 64
 #endif

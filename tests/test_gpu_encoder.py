@@ -279,12 +279,20 @@ def test_encoder_attention(ext, hip_device, seq, heads, qscale):
     close_rel(np32(out), _attn_ref(qkv, heads))
 
 
-@pytest.mark.parametrize('m,heads', [(1500, 20), (77, 20), (1, 20), (65, 20), (97, 20), (130, 20), (251, 20),
-                                     (1500, 2), (800, 4), (500, 6), (333, 8), (333, 10), (251, 12)])
-def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m, heads):
+@pytest.mark.parametrize('m', [1500, 77, 1, 65, 97, 130, 251])
+def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m):
     """The fused q/k/v projection writes the FW_EPI_SCALE_Q GEMM's q and k columns and, for v, exactly
-    what fw_encoder_pack_vt makes of that GEMM's v columns (padding keys zero); with fewer heads on either side
-    of where 64 x 64 tiles give way to 64 x 128."""
+    what fw_encoder_pack_vt makes of that GEMM's v columns (padding keys zero)."""
+    _check_qkv_against_gemm_and_pack(ext, hip_device, m, 20)
+
+
+@pytest.mark.parametrize('m,heads', [(1500, 2), (800, 4), (500, 6), (333, 8), (333, 10), (251, 12)])
+def test_encoder_qkv_of_fewer_heads(ext, hip_device, m, heads):
+    """The same on either side of where 64 x 64 tiles give way to 64 x 128 with fewer heads."""
+    _check_qkv_against_gemm_and_pack(ext, hip_device, m, heads)
+
+
+def _check_qkv_against_gemm_and_pack(ext, hip_device, m, heads):
     dev, d = hip_device, 64 * heads
     rng = np.random.default_rng(m)
     y = h16(np.float16(rng.standard_normal((m, d))), dev)
@@ -302,12 +310,20 @@ def test_encoder_qkv_matches_gemm_and_pack(ext, hip_device, m, heads):
     assert torch.equal(vt, vt_ref)
 
 
-# 256 x 256 tiles first, whole and partial last row tiles, then each of the others: 32 x 32, 64 x 32, 64 x 64,
-# 64 x 128, 128 x 128, 192 x 128, 256 x 128
-@pytest.mark.parametrize('t,layers', [(1500, 4), (1025, 3), (1281, 4), (50, 1), (100, 1), (251, 1), (100, 4), (251, 4),
-                                      (400, 4), (577, 4)])
-def test_cross_kv_matches_gemm(ext, hip_device, t, layers):
-    """The bits of the plain product, whose tiles add the same terms in the same order, in the cache layout."""
+@pytest.mark.parametrize('t,layers', [(1500, 4), (1025, 3), (1281, 4)])
+def test_cross_kv_wide_tiles_match_gemm(ext, hip_device, t, layers):
+    """Sizes that take the 256 x 256 tiles (whole and partial last row tiles): the bits of the plain product,
+    whose tiles add the same terms in the same order, in the cache layout."""
+    _check_cross_kv_against_gemm(ext, hip_device, t, layers)
+
+
+# one decoder layer: 32 x 32, 64 x 32 and 64 x 64 tiles; four: 64 x 128, 128 x 128, 192 x 128, 256 x 128
+@pytest.mark.parametrize('t,layers', [(50, 1), (100, 1), (251, 1), (100, 4), (251, 4), (400, 4), (577, 4)])
+def test_cross_kv_other_tiles_match_gemm(ext, hip_device, t, layers):
+    _check_cross_kv_against_gemm(ext, hip_device, t, layers)
+
+
+def _check_cross_kv_against_gemm(ext, hip_device, t, layers):
     rng = np.random.default_rng(t)
     enc = h16(rng.standard_normal((t, 1280)), hip_device)
     n = layers * 2 * 1280
